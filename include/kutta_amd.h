@@ -141,6 +141,14 @@ int ka_solver_host_waits(void* solver);
  * *level receives the level in use, 0 for none. No reference counterpart: the
  * iterates are those of the per-level launches either way. */
 int ka_solver_set_tail(void* solver, int first, int32_t* level);
+/* First AMG level of the multi-workgroup V-cycle (KH_GRID_CYCLE), which takes
+ * the automatic tail's place where its plan fits: first < 0 picks it
+ * automatically (the default), 0 turns it off, k >= 1 requests level k (an
+ * error if levels k.. do not fit; needs the tail automatic, which it sets).
+ * limit_us: how long its workgroups wait for each other before one of them
+ * works alone (default 2000). *level receives the level in use, 0 for none.
+ * No reference counterpart: identical iterates either way. */
+int ka_solver_set_grid(void* solver, int first, int limit_us, int32_t* level);
 /* The tail autotuner: times `repeats` V-cycles on the refreshed operator for
  * each admissible first level (and none) and keeps the fastest in *level.
  * The iterates are identical whichever is chosen. No reference counterpart. */

@@ -384,6 +384,19 @@ typedef enum kh_kernel {
      arguments, same bits), for levels with long rows. */
   KH_CSR_RESIDUAL_ROWWAVE,
   KH_PROLONG_SMOOTH_ROWWAVE,
+  /* The V-cycle (linalg/amg.cpp:283-310, no nullspace) from one level down in
+     one launch of several workgroups (no reference counterpart; bitwise the
+     per-level launches). INIT prepares a control block (ctl: KH_GRID_CTL_WORDS
+     words) on the device, once, before its first CYCLE; launches that share a
+     block must be ordered. CYCLE runs `count` levels (at most 16) over `parts`
+     workgroups as `table` says (parts x count kh_grid_part); levels [grid,
+     count), of at most KH_GRID_BOTTOM_ROWS rows each, belong to the first
+     workgroup alone. limit_us: how long workgroups wait for each other before
+     one of them does the whole cycle alone (0: at once).
+     levels,table,ctl,count,grid,pre,post,coarse_sweeps,parts,lds_words,
+     limit_us,rhs,out,status (n = 1). */
+  KH_GRID_INIT,                  /* ctl (n = 1) */
+  KH_GRID_CYCLE,
   KH_KERNEL_COUNT_MARK
 } kh_kernel;
 #define KH_COARSE_SWEEPS_MAX_ROWS 16384
@@ -447,6 +460,57 @@ typedef struct kh_tail_level {
  * swept (row starts, columns, values, l1 inverse, aggregate map), copied in on
  * each visit. */
 #define KH_TAIL_POOL_WORDS 40448
+
+/* KH_GRID_CYCLE's tables, as host/grid_plan.hpp builds them. A level: its
+ * operator, l1 inverse and transfer to the next level (as kh_tail_level); its
+ * iterate x, scratch w and right-hand side b (rows floats each; the first
+ * level's x and b are the launch's out and rhs); and the layout its members
+ * stage: place, the first slot (within its member) of each row, which takes
+ * KH_GRID_CHUNKS(its length in chunks of 4, rounded up) chunks of 4 slots;
+ * slot, the entry of each slot (-1 for padding); local_col, the slot's column
+ * within its member's window (0xffff for padding). */
+typedef struct kh_grid_level {
+  const int32_t* row_ptr;
+  const int32_t* col;
+  const float* val;
+  const float* inverse;
+  const int32_t* member_offsets;
+  const int32_t* members;
+  const int32_t* aggregate;
+  const uint16_t* place;
+  const int32_t* slot;
+  const uint16_t* local_col;
+  float* x;
+  float* w;
+  float* b;
+  int32_t rows;
+  int32_t pad;
+} kh_grid_level;
+/* One member's share of one level: rows [first, first + rows), the columns
+ * [window, window + window_rows) they read (its own rows among them), the
+ * slots [slot0, slot0 + slots), how a sweep sums its rows (mode: 0 entry by
+ * entry, 1 products formed first), and where in LDS (32-bit words) its share and the terms lie (the window
+ * takes the words before the terms) and, for the first level that is the first
+ * workgroup's alone, that workgroup's iterates. */
+typedef struct kh_grid_part {
+  int32_t first;
+  int32_t rows;
+  int32_t window;
+  int32_t window_rows;
+  int32_t slot0;
+  int32_t slots;
+  int32_t mode;
+  int32_t lds;
+  int32_t terms;
+  int32_t iterates;
+} kh_grid_part;
+#define KH_GRID_MAX_PARTS 32
+#define KH_GRID_BOTTOM_ROWS 256
+/* Chunks a row of `chunks` takes: an odd number when long, so that the rows of
+ * neighbouring lanes start on different LDS banks. */
+#define KH_GRID_CHUNKS(chunks) ((chunks) > 3 ? (chunks) | 1 : (chunks))
+#define KH_GRID_CTL_WORDS 128
+#define KH_GRID_POOL_WORDS 39936
 
 /* Device::launch (device.hpp:205; cuda_device.cu:132-140): runs kernel `kernel`
  * for global indices [0, n). n == 0 is a no-op; n > INT32_MAX, an unknown id or

@@ -122,6 +122,7 @@ def host_lib() -> C.CDLL:
         lib.ka_solver_set_fused.argtypes = [vp, i32]
         lib.ka_solver_host_waits.argtypes = [vp]
         lib.ka_solver_set_tail.argtypes = [vp, i32, pi32]
+        lib.ka_solver_set_grid.argtypes = [vp, i32, i32, pi32]
         lib.ka_solver_set_restart.argtypes = [vp, i32]
         lib.ka_solver_set_direct.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_dense_tolerance.argtypes = [vp, dbl]
@@ -402,6 +403,8 @@ class Kernel(enum.IntEnum):
     coarse_sweeps_resident = 256
     csr_residual_rowwave = 257
     prolong_smooth_rowwave = 258
+    grid_init = 259
+    grid_cycle = 260
 
 
 class Buffer:
@@ -900,6 +903,14 @@ class LinearSolver:
         0 off, k >= 1 level k. Returns the level in use (0: none)."""
         level = C.c_int32(0)
         _check_host(host_lib().ka_solver_set_tail(self.handle, int(first), C.byref(level)))
+        return level.value
+
+    def set_grid(self, first: int = -1, limit_us: int = 2000) -> int:
+        """First level of the multi-workgroup V-cycle: -1 automatic, 0 off,
+        k >= 1 level k; its workgroups wait limit_us for each other before one
+        works alone. Returns the level in use (0: none)."""
+        level = C.c_int32(0)
+        _check_host(host_lib().ka_solver_set_grid(self.handle, int(first), int(limit_us), C.byref(level)))
         return level.value
 
     def __del__(self):

@@ -308,5 +308,11 @@ int ka_solver_set_tail(void* s, int first, int* level) {
     if (level) *level = used;
   });
 }
+int ka_solver_set_grid(void* s, int first, int limit_us, int32_t* level) {
+  return guard([&] {
+    const int used = static_cast<Solver*>(s)->solver.set_grid(first, limit_us);
+    if (level) *level = used;
+  });
+}
 
 }  // extern "C"

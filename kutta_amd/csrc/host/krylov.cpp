@@ -19,6 +19,7 @@
 #include <iomanip>
 #include <sstream>
 
+#include "grid_plan.hpp"
 #include "learned.hpp"
 
 namespace kutta_amd {
@@ -108,6 +109,21 @@ struct KrylovSolver::Impl {
   int tail_request = -1;
   int tail_first = 0;
   DeviceArray<kh_tail_level> tail_table;
+  // The multi-workgroup V-cycle: levels [grid_first, end) run as one
+  // KH_GRID_CYCLE launch (0: off), in place of the tail, when the tail is
+  // automatic. grid_request < 0 picks the level by the rule in pick_grid.
+  int grid_request = -1;
+  int grid_first = 0;
+  int grid_limit_us = 2000;  // how long its workgroups wait for each other
+  GridPlan grid_plan;
+  struct GridLevelArrays {
+    DeviceArray<Index> slot;
+    DeviceArray<std::uint16_t> place, local_col;
+  };
+  std::vector<GridLevelArrays> grid_arrays;
+  DeviceArray<kh_grid_level> grid_levels;
+  DeviceArray<kh_grid_part> grid_table;
+  DeviceArray<std::uint32_t> grid_ctl;
 
   Impl(HipDevice& d, SolverKind k, const CsrHost& a, const AmgOptions& o)
       : dev(d), kind(k), options(o),
@@ -513,6 +529,7 @@ struct KrylovSolver::Impl {
     drop_graphs();
     tail_first = 0;
     tail_table = DeviceArray<kh_tail_level>();
+    drop_grid();
     if (!amg || tail_request == 0 || direct_level > 0) return;
     if (tail_request > 0) {
       KA_REQUIRE(tail_fits(std::size_t(tail_request)),
@@ -524,10 +541,13 @@ struct KrylovSolver::Impl {
           tail_first = int(i);
           break;
         }
+      pick_grid();
     }
-    if (tail_first == 0) return;
+    if (tail_first > 0) tail_table = to_device(dev, tail_levels(std::size_t(tail_first)));
+  }
+  std::vector<kh_tail_level> tail_levels(std::size_t first) const {
     std::vector<kh_tail_level> table;
-    for (std::size_t i = std::size_t(tail_first); i < levels.size(); ++i) {
+    for (std::size_t i = first; i < levels.size(); ++i) {
       const Level& l = levels[i];
       const DeviceCsr m = l.matrix.view();
       kh_tail_level t{};
@@ -545,7 +565,95 @@ struct KrylovSolver::Impl {
       t.nnz = l.nnz;
       table.push_back(t);
     }
-    tail_table = to_device(dev, table);
+    return table;
+  }
+
+  // ---- the multi-workgroup V-cycle (KH_GRID_CYCLE)
+  // By itself it takes over from the first level, at least two before the end,
+  // whose plan fits the LDS of 16 workgroups. Whole solves of tetrahedral
+  // pressure problems, V(5,5), ms:
+  //     first level's rows           none  tail only   8      16      32
+  //     1.0M cells, 17,004          18.34    18.34     -       -    16.86
+  //                  5,023                             -    17.03   17.35
+  //                  2,017                           17.19  17.24   17.54
+  //     78k cells,  19,808           5.75     5.81     -       -     5.15
+  //                  5,138                            5.03   5.01    5.21
+  //     10k cells,   2,611           4.59     3.97    2.63   2.64    2.69
+  //                    681                            2.94   2.92    2.96
+  // so 8 or 16 workgroups do alike, and 32, which hold more, pay only where the
+  // autotuner finds so or a caller asks. A last level by itself (15,292 rows, 4
+  // sweeps a visit under a K-cycle) took 19.25 against 18.81.
+  static constexpr Index kGridAutoRows = 24576;
+  static constexpr int kGridParts = 16;
+  bool grid_allowed(std::size_t first) const {
+    return amg && !nullspace && !coarse_bf16 && direct_level == 0 && first >= tail_floor() && first < levels.size() &&
+           levels[first].rows <= kGridAutoRows && levels[first].rows > KH_GRID_BOTTOM_ROWS;
+  }
+  bool plan_grid_at(std::size_t first, GridPlan& plan, bool automatic = false) const {
+    if (!grid_allowed(first)) return false;
+    std::vector<const CsrHost*> patterns;
+    for (std::size_t i = first; i < levels.size(); ++i) patterns.push_back(&levels[i].host);
+    return plan_grid(patterns, kGridParts, plan) || (!automatic && plan_grid(patterns, KH_GRID_MAX_PARTS, plan));
+  }
+  void drop_grid() {
+    grid_first = 0;
+    grid_arrays.clear();
+    grid_levels = DeviceArray<kh_grid_level>();
+    grid_table = DeviceArray<kh_grid_part>();
+  }
+  void pick_grid() {
+    if (grid_request == 0) return;
+    if (grid_request > 0) {
+      if (plan_grid_at(std::size_t(grid_request), grid_plan)) use_grid(grid_request);
+      return;
+    }
+    for (std::size_t i = 1; i + 1 < levels.size(); ++i)
+      if (plan_grid_at(i, grid_plan, true)) {
+        use_grid(int(i));
+        return;
+      }
+  }
+  // Uploads grid_plan's tables for levels [first, end).
+  void use_grid(int first) {
+    std::vector<kh_grid_level> table;
+    grid_arrays.clear();
+    for (std::size_t i = std::size_t(first); i < levels.size(); ++i) {
+      const Level& l = levels[i];
+      const DeviceCsr m = l.matrix.view();
+      kh_grid_level g{};
+      g.row_ptr = m.row_ptr;
+      g.col = m.col;
+      g.val = m.val;
+      g.inverse = l.l1.data();
+      if (l.has_transfer) {
+        g.member_offsets = l.member_offsets.data();
+        g.members = l.members.data();
+        g.aggregate = l.aggregate.data();
+      }
+      const GridLevelPlan& p = grid_plan.levels[i - std::size_t(first)];
+      grid_arrays.push_back({to_device(dev, p.slot), to_device(dev, p.place), to_device(dev, p.local_col)});
+      g.place = grid_arrays.back().place.data();
+      g.slot = grid_arrays.back().slot.data();
+      g.local_col = grid_arrays.back().local_col.data();
+      g.x = l.x.data();
+      g.w = l.r.data();
+      g.b = l.b.data();
+      g.rows = l.rows;
+      table.push_back(g);
+    }
+    grid_levels = to_device(dev, table);
+    grid_table = to_device(dev, grid_plan.table);
+    if (grid_ctl.empty()) {
+      grid_ctl = DeviceArray<std::uint32_t>(dev, KH_GRID_CTL_WORDS);
+      dev.launch(KH_GRID_INIT, 1, {grid_ctl});
+    }
+    grid_first = first;
+  }
+  void grid_cycle(const float* b, float* x, const int* st) {
+    dev.launch(KH_GRID_CYCLE, 1,
+               {grid_levels, grid_table, grid_ctl, grid_plan.count, grid_plan.grid, options.pre_sweeps,
+                options.post_sweeps, options.coarse_sweeps, grid_plan.parts, grid_plan.lds_words, grid_limit_us, b, x,
+                st});
   }
 
   DeviceCsr level_operator(std::size_t i, const DeviceCsr& fine) const {
@@ -699,7 +807,12 @@ struct KrylovSolver::Impl {
     Level& l = levels[index];
     float* w = l.r.data();
     CycleResult result;
-    if (fused && tail_first > 0 && int(index) == tail_first) {
+    const bool grid = grid_first > 0 && !coarse_bf16;
+    if (fused && grid && int(index) == grid_first) {
+      grid_cycle(b, x, st);
+      return result;
+    }
+    if (fused && !grid && tail_first > 0 && int(index) == tail_first) {
       dev.launch(KH_FUSED_COARSE_TAIL, 1,
                  {tail_table, int(levels.size() - index), options.pre_sweeps, options.post_sweeps,
                   options.coarse_sweeps, nullspace ? 1 : 0, b, x, st});
@@ -1351,6 +1464,7 @@ std::vector<SolveStats> KrylovSolver::solve_batched(const std::vector<KrylovSolv
 int KrylovSolver::set_tail(int first) {
   const int previous = impl_->tail_request;
   impl_->tail_request = first;
+  if (first < 0) impl_->grid_request = -1;
   try {
     impl_->plan_tail();
   } catch (...) {
@@ -1361,6 +1475,20 @@ int KrylovSolver::set_tail(int first) {
   return impl_->tail_first;
 }
 int KrylovSolver::tail_level() const { return impl_->tail_first; }
+int KrylovSolver::set_grid(int first, int limit_us) {
+  Impl& I = *impl_;
+  KA_REQUIRE(limit_us >= 0, "AMG: the multi-workgroup cycle's wait must not be negative");
+  if (first > 0) {
+    GridPlan plan;
+    KA_REQUIRE(I.plan_grid_at(std::size_t(first), plan),
+               "AMG: levels from " + std::to_string(first) + " do not fit the multi-workgroup cycle");
+  }
+  I.grid_request = first;
+  I.grid_limit_us = limit_us;
+  if (first != 0) I.tail_request = -1;
+  I.plan_tail();
+  return I.grid_first;
+}
 
 // The coarse-tail autotuner (no reference counterpart): times `repeats`
 // V-cycles for each admissible first level of the tail, and for none, keeps
@@ -1517,6 +1645,23 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
       best = first;
     }
   }
+  // The multi-workgroup cycle from each level whose plan fits, in the tail's place.
+  int best_grid = 0;
+  for (std::size_t i = 1; i < I.levels.size(); ++i) {
+    if (!I.grid_allowed(i)) continue;
+    I.tail_request = -1;
+    I.grid_request = int(i);
+    I.plan_tail();
+    if (I.grid_first == 0) continue;
+    I.reset(0);
+    const double secs = seconds([&] { I.apply(a, v.data(), out.data(), Tail::None); });
+    if (secs < kKeep * best_s) {
+      best_s = secs;
+      best = -1;
+      best_grid = int(i);
+    }
+  }
+  I.grid_request = best_grid;
   I.tail_request = best;
   I.plan_tail();
   return I.tail_first;
@@ -1642,6 +1787,9 @@ std::string KrylovSolver::plan() const {
             : impl_->coarse_sweeps_mode == 2 && L.back().resident_cap > 0 ? "register-resident sweeps"
                                                                             : "one-workgroup sweeps");
   out << "; tail from level " << impl_->tail_first;
+  if (impl_->grid_first > 0)
+    out << ", multi-workgroup cycle from level " << impl_->grid_first << " (" << impl_->grid_plan.parts
+        << " workgroups)";
   out << "; longest row per level";
   for (std::size_t i = 0; i < L.size(); ++i) out << (i ? "," : " ") << L[i].max_row;
   out << "; sweeps per level";

@@ -98,6 +98,11 @@ class KrylovSolver {
   // Returns the level in use (0: none).
   int set_tail(int first);
   int tail_level() const;
+  // The multi-workgroup V-cycle (KH_GRID_CYCLE): first < 0 picks its first
+  // level automatically (the default), 0 turns it off, k requests level k;
+  // limit_us is how long its workgroups wait for each other before one works
+  // alone. Returns the level in use, 0 for none (iterates are the same).
+  int set_grid(int first, int limit_us);
   // Times `repeats` V-cycles per admissible tail level (and none) on the
   // refreshed operator and keeps the fastest; returns it. Identical iterates
   // either way. No reference counterpart.

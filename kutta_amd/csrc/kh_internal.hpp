@@ -43,6 +43,7 @@ struct kh_device {
   double* results = nullptr;
   double* results_host = nullptr;
   bool capturing = false;
+  bool grid_ready = false;  // the multi-workgroup V-cycle's LDS limit is set on this device
   std::vector<kh::ProfileSlot> profile;
   // Events for the next packet-timed launch (null when not profiling it).
   hipEvent_t packet_start = nullptr;
@@ -90,6 +91,7 @@ const std::vector<KernelEntry>& gmres_kernels();
 const std::vector<KernelEntry>& dense_kernels();
 const std::vector<KernelEntry>& learned_kernels();
 const std::vector<KernelEntry>& fv_kernels();
+const std::vector<KernelEntry>& grid_kernels();
 
 // Reduction launchers (kh_reduce.hip).
 void launch_reduce_into(kh_device* dev, int mode, const float* x, const float* y,
