@@ -271,7 +271,7 @@ typedef enum kh_kernel {
      reference counterpart); the operator must be symmetric positive definite. */
   KH_DENSE_INVERT,               /* blocked Gauss-Jordan inverse of an n-row CSR operator, FP64 (the
                                     panel and update products on the FP64 MFMA), no pivoting:
-                                    rows,cols,values,inverse (n*n doubles),scratch (4096 doubles);
+                                    rows,cols,values,inverse (n*n doubles),scratch (not used);
                                     n <= 8192 */
   KH_DENSE_APPLY,                /* x = inverse b (FP64 accumulation): inverse,b,x,status */
   /* Learned coarse correction (no reference counterpart): a message-passing

@@ -4,7 +4,7 @@
 // Gauss-Jordan elimination without pivoting (the operator is symmetric
 // positive definite: a pinned M-matrix and its Galerkin products). Per block
 // of kGjBlock pivots K:
-//   P = A_KK^-1 (one workgroup, element-wise Gauss-Jordan in LDS), A_KK = P
+//   P = A_KK^-1 (one workgroup, element-wise Gauss-Jordan), A_KK = P
 //   A_KJ = P A_KJ                (row panel, J outside K)
 //   A_IJ -= A_IK A_KJ            (trailing update, I and J outside K)
 //   A_IK = -A_IK P               (column panel)
@@ -18,7 +18,7 @@ namespace {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kGjBlock = 64;          // pivots per block, and the tile edge
-constexpr int kGjStride = kGjBlock + 1;  // LDS row stride (doubles), padded
+constexpr int kGjStride = kGjBlock + 2;  // LDS row stride (doubles): half a wavefront's L operands fall on all banks
 
 __global__ void __launch_bounds__(kBlock) k_dense_clear(long count, double* __restrict__ dense) {
   const long i = long(blockIdx.x) * kBlock + threadIdx.x;
@@ -31,118 +31,195 @@ __global__ void __launch_bounds__(kBlock) k_dense_scatter(int n, const int* __re
   for (int j = rows[i]; j < rows[i + 1]; ++j) dense[long(i) * n + cols[j]] += double(values[j]);
 }
 
-// P = A_KK^-1 for K = [k0, k0 + b): element-wise Gauss-Jordan on the block in
-// LDS, pivot by pivot with the pivot's reciprocal r = 1/p (a_pp' = r,
-// a_pj' = a_pj r, a_ip' = -a_ip r, a_ij' = a_ij - a_ip (a_pj r)); written to
-// P (kGjBlock x kGjBlock) and A_KK. One 1024-thread workgroup, four entries
-// per thread.
-constexpr int kGjPivotThreads = 1024;
-__global__ void __launch_bounds__(kGjPivotThreads) k_gj_pivot(int n, int k0, int b, double* __restrict__ a,
-                                                              double* __restrict__ p) {
-  __shared__ double t[kGjBlock * kGjStride];
-  __shared__ double row[kGjBlock], col[kGjBlock];
-  for (int e = threadIdx.x; e < b * b; e += kGjPivotThreads) {
-    const int i = e / b, j = e % b;
-    t[i * kGjStride + j] = a[long(k0 + i) * n + k0 + j];
+// A 64 x 64 tile on one 256-thread workgroup: thread (wave w, lane l) holds
+// column 16 w + l % 16 and the rows of its 16 slots, slot m being row
+// 4 m + l / 16. That is the accumulator of v_mfma_f64_16x16x4_f64 (register q
+// of row block br is slot 4 br + q: the FP64 accumulator interleaves rows;
+// checked against a CPU product on the device), for which the lane supplies
+// L[16 br + l%16][4 s + l/16] and R[4 s + l/16][16 w + l%16]: a tile's R comes
+// from memory straight into that layout, L through LDS.
+constexpr int kSlots = 16;
+__device__ __forceinline__ int tile_row(int m) { return 4 * m + ((threadIdx.x & 63) >> 4); }
+__device__ __forceinline__ int tile_col() { return 16 * int(threadIdx.x >> 6) + int(threadIdx.x & 15); }
+// The tile at (i0, j0), zero from `rows` and `cols` on. All 16 loads are in
+// flight before the first is used.
+__device__ __forceinline__ void load_slots(double (&v)[kSlots], const double* __restrict__ a, int n, int i0, int j0,
+                                           int rows, int cols) {
+  const int c = tile_col();
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    v[m] = a[long(i0 + min(tile_row(m), rows - 1)) * n + j0 + min(c, cols - 1)];
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    if (tile_row(m) >= rows || c >= cols) v[m] = 0.0;
+}
+// The tile as the left factor: consecutive threads load consecutive columns.
+__device__ __forceinline__ void load_rows(double (&v)[kSlots], const double* __restrict__ a, int n, int i0, int j0,
+                                          int rows, int cols) {
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    v[m] = a[long(i0 + min(r0 + 4 * m, rows - 1)) * n + j0 + min(c, cols - 1)];
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    if (r0 + 4 * m >= rows || c >= cols) v[m] = 0.0;
+}
+__device__ __forceinline__ void stage_rows(double* L, const double (&v)[kSlots]) {
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m) L[(r0 + 4 * m) * kGjStride + c] = v[m];
+}
+// L R for the staged L and this thread's R values.
+__device__ __forceinline__ void tile_product(const double* L, const double (&rv)[kSlots], double (&out)[kSlots]) {
+  const int lane = threadIdx.x & 63;
+  const double* l = L + (lane & 15) * kGjStride + (lane >> 4);
+  f64x4 acc[4] = {};
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+#pragma unroll
+    for (int br = 0; br < 4; ++br)
+      acc[br] = __builtin_amdgcn_mfma_f64_16x16x4f64(l[16 * br * kGjStride + 4 * s], rv[s], acc[br], 0, 0, 0);
   }
-  __syncthreads();
-  for (int q = 0; q < b; ++q) {
-    const double r = 1.0 / t[q * kGjStride + q];
-    if (threadIdx.x < b) {
-      row[threadIdx.x] = t[q * kGjStride + threadIdx.x] * r;  // the new pivot row (a_qj r)
-      col[threadIdx.x] = t[threadIdx.x * kGjStride + q];
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m) out[m] = acc[m / 4][m % 4];
+}
+__device__ __forceinline__ void store_slots(const double (&v)[kSlots], double* __restrict__ a, int n, int i0, int j0,
+                                            int rows, int cols) {
+  const int c = tile_col();
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    if (tile_row(m) < rows && c < cols) a[long(i0 + tile_row(m)) * n + j0 + c] = v[m];
+}
+
+// The inverse of the b x b tile held in slots: element-wise Gauss-Jordan,
+// pivot by pivot with the pivot's reciprocal r = 1/p (a_pp' = r,
+// a_pj' = a_pj r, a_ip' = -a_ip r, a_ij' = a_ij - a_ip (a_pj r)). Rows and
+// columns from b on are taken as the identity's, which leaves the rest as it
+// is. A pivot is one barrier: its row and column go out through LDS (two
+// buffers in turn) and every thread forms r itself. The slots turn by one
+// every four pivots, so that the pivot's row is always in slot 0 and no
+// register is indexed at run time. 64 pivots: 80 us before (four entries of
+// 1024 threads in LDS, two barriers each, and a launch of its own).
+__device__ __forceinline__ void invert_slots(double (&t)[kSlots], int b, double* lds) {
+  const int lane = threadIdx.x & 63, sub = lane >> 4, j = tile_col();
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m)
+    if (tile_row(m) >= b || j >= b) t[m] = tile_row(m) == j ? 1.0 : 0.0;
+  for (int group = 0; group < kSlots; ++group) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = 4 * group + u;
+      double* row = lds + (u & 1) * 2 * kGjBlock;
+      double* col = row + kGjBlock;  // [sub][slot]
+      if (sub == u) row[j] = t[0];
+      if (j == q) {
+#pragma unroll
+        for (int m = 0; m < kSlots; ++m) col[sub * kSlots + m] = t[m];
+      }
+      __syncthreads();
+      const double r = 1.0 / row[q], scaled = row[j] * r;
+      const bool mine = j == q;
+      double c[kSlots];
+#pragma unroll
+      for (int m = 0; m < kSlots; ++m) c[m] = col[sub * kSlots + m];
+#pragma unroll
+      for (int m = 0; m < kSlots; ++m) {
+        const double v = mine ? -c[m] * r : t[m] - c[m] * scaled;
+        t[m] = m == 0 && sub == u ? (mine ? r : scaled) : v;
+      }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < b * b; e += kGjPivotThreads) {
-      const int i = e / b, j = e % b;
-      double v;
-      if (i == q && j == q) v = r;
-      else if (i == q) v = row[j];
-      else if (j == q) v = -col[i] * r;
-      else v = t[i * kGjStride + j] - col[i] * row[j];
-      t[i * kGjStride + j] = v;
-    }
-    __syncthreads();
-  }
-  for (int e = threadIdx.x; e < kGjBlock * kGjBlock; e += kGjPivotThreads) {
-    const int i = e / kGjBlock, j = e % kGjBlock;
-    const double v = (i < b && j < b) ? t[i * kGjStride + j] : 0.0;
-    p[e] = v;
-    if (i < b && j < b) a[long(k0 + i) * n + k0 + j] = v;
+    const double first = t[0];
+#pragma unroll
+    for (int m = 0; m + 1 < kSlots; ++m) t[m] = t[m + 1];
+    t[kSlots - 1] = first;
   }
 }
 
-// The three panel and update products of one block step, 64 x 64 output
-// tiles of C = L R with L, R staged in LDS (zero outside the matrix and the
-// block). Wave w computes the 16 x 16 sub-blocks (w, 0..3); lane l of a
-// v_mfma_f64_16x16x4_f64 supplies L[16 br + l%16][4 s + l/16] and
-// R[4 s + l/16][16 bc + l%16] and its accumulator register q holds row
-// 4 q + l/16, column l % 16 (the FP64 accumulator interleaves rows; checked
-// against a CPU product on the device).
-enum class GjTile { Rows, Update, Cols };
-template <GjTile M>
-__global__ void __launch_bounds__(kBlock) k_gj_tile(int n, int k0, int b, double* __restrict__ a,
-                                                    const double* __restrict__ p) {
-  __shared__ double L[kGjBlock * kGjStride];
-  __shared__ double R[kGjBlock * kGjStride];
-  // Tile origin: Rows tiles columns, Cols tiles rows, Update tiles both.
-  int i0 = 0, j0 = 0;
-  if constexpr (M == GjTile::Rows) j0 = int(blockIdx.x) * kGjBlock;
-  if constexpr (M == GjTile::Cols) i0 = int(blockIdx.x) * kGjBlock;
-  if constexpr (M == GjTile::Update) {
-    i0 = int(blockIdx.y) * kGjBlock;
-    j0 = int(blockIdx.x) * kGjBlock;
-    if (i0 == k0 || j0 == k0) return;  // whole tile inside the block's rows or columns
+// The trailing update of block k0 (none if k0 < 0), one workgroup per tile.
+// The tile of the next block's pivots goes first and is inverted on the way,
+// behind the other tiles' work.
+// What bounds it: at 3,375 rows 91 MB read and 91 MB written per block (27 us
+// at the rate of a copy of that size) beside 64 FP64 MFMA of 64 cycles per
+// wave and tile (19 us); it takes 51 us. At 8,000 rows it moves 3.9 TB/s, a
+// copy 4.7. All of a tile's 48 loads per thread are in flight together, and
+// three workgroups fit a CU. The whole inverse takes 3.3 ms at 3,375 rows and
+// 33.7 at 8,000; with a load at a time per thread and four launches a block it
+// took 10.8 and 91.7.
+__global__ void __launch_bounds__(kBlock, 3) k_gj_update(int n, int k0, double* __restrict__ a) {
+  __shared__ __align__(16) double L[kGjBlock * kGjStride];
+  const int tiles = (n + kGjBlock - 1) / kGjBlock, block = k0 < 0 ? -1 : k0 / kGjBlock, next = block + 1;
+  // Tile number `first` and tile 0 change places.
+  const int first = next * tiles + next;
+  int tile = int(blockIdx.x);
+  if (next < tiles) tile = tile == 0 ? first : tile == first ? 0 : tile;
+  const int ti = tile / tiles, tj = tile % tiles;
+  if (ti == block || tj == block) return;
+  const int i0 = ti * kGjBlock, j0 = tj * kGjBlock;
+  const int rows = min(kGjBlock, n - i0), cols = min(kGjBlock, n - j0);
+  double c[kSlots];
+  if (k0 >= 0) {
+    double l[kSlots], r[kSlots], product[kSlots];
+    const int b = min(kGjBlock, n - k0);
+    load_rows(l, a, n, i0, k0, rows, b);
+    load_slots(r, a, n, k0, j0, b, cols);
+    load_slots(c, a, n, i0, j0, rows, cols);
+    stage_rows(L, l);
+    __syncthreads();
+    tile_product(L, r, product);
+#pragma unroll
+    for (int m = 0; m < kSlots; ++m) c[m] -= product[m];
+  } else {
+    load_slots(c, a, n, i0, j0, rows, cols);
   }
-  if constexpr (M == GjTile::Rows) {
-    if (j0 == k0) return;
+  if (ti == next && tj == next) {
+    __syncthreads();
+    invert_slots(c, rows, L);
   }
-  if constexpr (M == GjTile::Cols) {
-    if (i0 == k0) return;
+  store_slots(c, a, n, i0, j0, rows, cols);
+}
+
+// Between the updates of two blocks: the column panel of block k0 (none if
+// k0 < 0), A_IK = -A_IK P (blockIdx.y 0), and the row panel of the next block
+// K' (none after the last), A_K'J = P' A_K'J (blockIdx.y 1). The one tile that
+// both panels share, A_K'K, takes both steps in the second.
+__global__ void __launch_bounds__(kBlock, 3) k_gj_panels(int n, int k0, double* __restrict__ a) {
+  __shared__ __align__(16) double L[kGjBlock * kGjStride];
+  const int block = k0 < 0 ? -1 : k0 / kGjBlock, next = block + 1, t = int(blockIdx.x), t0 = t * kGjBlock;
+  const int k1 = next * kGjBlock, b0 = k0 < 0 ? 0 : min(kGjBlock, n - k0), b1 = min(kGjBlock, n - k1);
+  const int extent = min(kGjBlock, n - t0);
+  double l[kSlots], r[kSlots], v[kSlots];
+  if (blockIdx.y == 0) {
+    if (k0 < 0 || t == block || t == next) return;
+    load_rows(l, a, n, t0, k0, extent, b0);
+    load_slots(r, a, n, k0, k0, b0, b0);
+    stage_rows(L, l);
+    __syncthreads();
+    tile_product(L, r, v);
+#pragma unroll
+    for (int m = 0; m < kSlots; ++m) v[m] = -v[m];
+    store_slots(v, a, n, t0, k0, extent, b0);
+    return;
   }
-  for (int e = threadIdx.x; e < kGjBlock * kGjBlock; e += kBlock) {
-    const int r = e / kGjBlock, c = e % kGjBlock;
-    double lv = 0.0, rv = 0.0;
-    if constexpr (M == GjTile::Rows) {
-      lv = p[e];  // zero outside b x b
-      if (r < b && j0 + c < n) rv = a[long(k0 + r) * n + j0 + c];
-    } else if constexpr (M == GjTile::Update) {
-      if (i0 + r < n && c < b) lv = a[long(i0 + r) * n + k0 + c];
-      if (r < b && j0 + c < n) rv = a[long(k0 + r) * n + j0 + c];
-    } else {
-      if (i0 + r < n && c < b) lv = a[long(i0 + r) * n + k0 + c];
-      rv = p[e];
-    }
-    L[r * kGjStride + c] = lv;
-    R[r * kGjStride + c] = rv;
+  if (b1 <= 0 || t == next) return;
+  double p[kSlots];
+  load_rows(p, a, n, k1, k1, b1, b1);
+  if (t == block) {
+    load_rows(l, a, n, k1, k0, b1, b0);
+    load_slots(r, a, n, k0, k0, b0, b0);
+    stage_rows(L, l);
+    __syncthreads();
+    tile_product(L, r, v);
+    // The MFMA's right factor has slot s's row in s: the accumulator's layout.
+#pragma unroll
+    for (int m = 0; m < kSlots; ++m) r[m] = -v[m];
+    __syncthreads();
+  } else {
+    load_slots(r, a, n, k1, t0, b1, extent);
   }
+  stage_rows(L, p);
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  f64x4 acc[4];
-#pragma unroll
-  for (int bc = 0; bc < 4; ++bc) acc[bc] = f64x4{0.0, 0.0, 0.0, 0.0};
-  for (int s = 0; s < kGjBlock / 4; ++s) {
-    const double lv = L[(16 * wave + (lane & 15)) * kGjStride + 4 * s + (lane >> 4)];
-#pragma unroll
-    for (int bc = 0; bc < 4; ++bc) {
-      const double rv = R[(4 * s + (lane >> 4)) * kGjStride + 16 * bc + (lane & 15)];
-      acc[bc] = __builtin_amdgcn_mfma_f64_16x16x4f64(lv, rv, acc[bc], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int bc = 0; bc < 4; ++bc) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = 16 * wave + 4 * q + (lane >> 4), c = 16 * bc + (lane & 15);
-      if constexpr (M == GjTile::Rows) {
-        if (r < b && j0 + c < n) a[long(k0 + r) * n + j0 + c] = acc[bc][q];
-      } else if constexpr (M == GjTile::Update) {
-        if (i0 + r < n && j0 + c < n) a[long(i0 + r) * n + j0 + c] -= acc[bc][q];
-      } else {
-        if (i0 + r < n && c < b) a[long(i0 + r) * n + k0 + c] = -acc[bc][q];
-      }
-    }
-  }
+  tile_product(L, r, v);
+  store_slots(v, a, n, k1, t0, b1, extent);
 }
 
 // x = inverse b in FP64, rounded to FP32; one workgroup per row.
@@ -162,23 +239,21 @@ __global__ void __launch_bounds__(kBlock) k_dense_apply(int n, const double* __r
 #define KD(k) static_cast<double*>(buf(a, k))
 
 // rows, cols, values, inverse, scratch (n = rows of the dense operator;
-// inverse n*n doubles, scratch at least kGjBlock^2): the dense inverse of the
-// CSR operator, left in `inverse`.
+// inverse n*n doubles; scratch is not used): the dense inverse of the CSR
+// operator, left in `inverse`.
 void l_dense_invert(kh_device* d, int n, const kh_arg* a) {
   if (n > 8192) throw std::runtime_error("dense_invert: at most 8192 rows");
   if (n < 1) return;
   const long count = long(n) * n;
   double* m = KD(3);
-  double* p = KD(4);
   k_dense_clear<<<dim3(unsigned((count + kBlock - 1) / kBlock)), dim3(kBlock), 0, d->stream>>>(count, m);
   k_dense_scatter<<<dim3(blocks_for(n)), dim3(kBlock), 0, d->stream>>>(n, KB(0), KB(1), KCF(2), m);
   const unsigned tiles = unsigned((n + kGjBlock - 1) / kGjBlock);
+  k_gj_update<<<dim3(1), dim3(kBlock), 0, d->stream>>>(n, -1, m);
+  k_gj_panels<<<dim3(tiles, 2), dim3(kBlock), 0, d->stream>>>(n, -1, m);
   for (int k0 = 0; k0 < n; k0 += kGjBlock) {
-    const int b = std::min(kGjBlock, n - k0);
-    k_gj_pivot<<<dim3(1), dim3(kGjPivotThreads), 0, d->stream>>>(n, k0, b, m, p);
-    k_gj_tile<GjTile::Rows><<<dim3(tiles), dim3(kBlock), 0, d->stream>>>(n, k0, b, m, p);
-    k_gj_tile<GjTile::Update><<<dim3(tiles, tiles), dim3(kBlock), 0, d->stream>>>(n, k0, b, m, p);
-    k_gj_tile<GjTile::Cols><<<dim3(tiles), dim3(kBlock), 0, d->stream>>>(n, k0, b, m, p);
+    if (tiles > 1) k_gj_update<<<dim3(tiles * tiles), dim3(kBlock), 0, d->stream>>>(n, k0, m);
+    k_gj_panels<<<dim3(tiles, 2), dim3(kBlock), 0, d->stream>>>(n, k0, m);
   }
 }
 // inverse, b, x, status

@@ -234,3 +234,26 @@ def test_lazy_dense_refresh(device):
     eager.refresh(m)
     ste, xe = solve(eager)
     assert st3.iterations == ste.iterations and np.array_equal(x3.view(np.uint32), xe.view(np.uint32))
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (63, 1, 1), (8, 8, 1), (5, 13, 1), (127, 1, 1), (8, 4, 4), (43, 3, 1),
+                                      (7, 7, 7)])
+def test_dense_inverse_stays_inside_its_matrix(device, nx, ny, nz):
+    """The block products at 1, 63, 64, 65, 127, 128, 129 and 343 rows with NaN
+    stored behind the matrix: nothing beyond the last partial block is
+    taken into a product or written. The bound is that of
+    test_blocked_gauss_jordan_inverse."""
+    a = oracle.poisson(nx, ny, nz, 1.0, random=True)
+    n, guard = a.n_rows, 64 * a.n_rows + 64
+    A = dense_of(a).astype(np.float32).astype(np.float64)
+    rows = device.upload(np.asarray(a.row_ptr, np.int32), np.int32)
+    cols = device.upload(np.asarray(a.col, np.int32), np.int32)
+    vals = device.upload(np.asarray(a.val, np.float32))
+    padded = device.upload(np.full(n * n + guard, np.nan).view(np.float32))
+    scratch = device.alloc(4096 * 2, np.float32)
+    device.launch(kutta_amd.Kernel.dense_invert, n, rows, cols, vals, padded, scratch)
+    got = padded.download().view(np.float64)
+    assert np.isnan(got[n * n:]).all()
+    got = got[:n * n].reshape(n, n)
+    cond = np.linalg.cond(A)
+    assert np.abs(got - np.linalg.inv(A)).max() <= 1e-13 * cond * np.abs(np.linalg.inv(A)).max()
