@@ -209,11 +209,10 @@ __device__ __forceinline__ double block_sum(double v, double* lds /* kBlock/64 *
   return total;
 }
 
-// Grid reductions are two launches: each workgroup stores its partial sums at
-// a fixed slot (no fences, no atomics), and a one-workgroup finisher sums the
-// slots in a fixed order after the kernel boundary has made them visible.
-// A device-scope fence per workgroup would write back and invalidate the L2 of
-// every XCD and costs far more than the second launch.
+// Grid reductions: each workgroup stores its partial sums at a fixed slot, and
+// one workgroup sums the slots in a fixed order, in a launch of its own after
+// the kernel boundary has made them visible, or as the last workgroup of the
+// same launch (last_workgroup).
 template <int N>
 __device__ __forceinline__ void store_partials(const double (&mine)[N], double* partials) {
   if (threadIdx.x == 0) {
@@ -221,16 +220,48 @@ __device__ __forceinline__ void store_partials(const double (&mine)[N], double* 
     for (int k = 0; k < N; ++k) partials[blockIdx.x * N + k] = mine[k];
   }
 }
+// Stores the workgroup's partials and returns, in all its threads, whether it
+// is the launch's last one, which may then read every slot (sum_partials with
+// kHere). No fence: that would write back and invalidate the L2 of every XCD.
+// The slots are written through it (agent-scope stores, waited for) before the
+// ticket is taken and read past it. Tickets are counted in kTicketGroups lines
+// and then over those, since one counter takes only some 10 ns an increment;
+// the last to take one leaves it zero for the next launch.
+constexpr unsigned kTicketGroups = 16, kTicketStride = 32;
+constexpr unsigned kTicketWords = (kTicketGroups + 1) * kTicketStride;
+template <int N>
+__device__ __forceinline__ bool last_workgroup(const double (&mine)[N], double* partials, unsigned* tickets) {
+  __shared__ int last;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      __hip_atomic_store(partials + blockIdx.x * N + k, mine[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const auto take = [](unsigned* t, unsigned count) {
+      if (__hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != count) return false;
+      __hip_atomic_store(t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return true;
+    };
+    const unsigned group = blockIdx.x % kTicketGroups, groups = min(gridDim.x, kTicketGroups);
+    last = take(tickets + (1 + group) * kTicketStride, (gridDim.x - group + kTicketGroups - 1) / kTicketGroups) &&
+           take(tickets, groups);
+  }
+  __syncthreads();
+  return last != 0;
+}
 // Finisher body: the totals of `count` partial slots, valid on thread 0. Each
 // thread adds slots threadIdx.x, +blockDim.x, ... in that order; the loads of
 // kSumAhead consecutive slots of a thread are issued before their adds, so
 // the finisher pays one memory round trip per kSumAhead slots instead of one
 // per slot (a few thousand partials at a million rows), with the same sums.
 constexpr int kSumAhead = 8;
-template <int N>
+template <int N, bool kHere = false>
 __device__ __forceinline__ void sum_partials(const double* partials, unsigned count,
                                              double (&total)[N]) {
   __shared__ double lds[N][kBlock / 64];
+  const auto load = [&](unsigned k) {
+    return kHere ? __hip_atomic_load(partials + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : partials[k];
+  };
   double v[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) v[k] = 0;
@@ -241,7 +272,7 @@ __device__ __forceinline__ void sum_partials(const double* partials, unsigned co
 #pragma unroll
     for (int u = 0; u < kSumAhead; ++u)
 #pragma unroll
-      for (int k = 0; k < N; ++k) p[u][k] = partials[(b + u * stride) * N + k];
+      for (int k = 0; k < N; ++k) p[u][k] = load((b + u * stride) * N + k);
 #pragma unroll
     for (int u = 0; u < kSumAhead; ++u)
 #pragma unroll
@@ -249,7 +280,7 @@ __device__ __forceinline__ void sum_partials(const double* partials, unsigned co
   }
   for (; b < count; b += stride)
 #pragma unroll
-    for (int k = 0; k < N; ++k) v[k] += partials[b * N + k];
+    for (int k = 0; k < N; ++k) v[k] += load(b * N + k);
 #pragma unroll
   for (int k = 0; k < N; ++k) total[k] = block_sum(v[k], lds[k]);
 }

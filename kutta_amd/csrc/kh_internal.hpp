@@ -37,8 +37,11 @@ struct kh_device {
   std::string name;
   hipStream_t stream = nullptr;
   // Reduction scratch: per-workgroup partial sums (two doubles per workgroup
-  // for the fused dot pair), consumed by a finisher launch.
+  // for the fused dot pair), summed by the launch's last workgroup or by a
+  // finisher launch; and the counters that find the last workgroup, one set
+  // per lane, zero between launches.
   double* partials = nullptr;
+  unsigned* tickets = nullptr;
   // Host reduction results: device staging and pinned host copy.
   double* results = nullptr;
   double* results_host = nullptr;

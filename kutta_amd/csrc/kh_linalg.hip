@@ -507,13 +507,93 @@ __global__ void k_solver_project(int n, float* __restrict__ x, const float* __re
 
 // ------------------------------------------------------------ fused kernels
 // A fused reduction is a row kernel that stores one FP64 partial per
-// workgroup (store_partials) and a one-workgroup finisher that sums the slots
-// in order and applies the scalar update of the reference sequence it replaces.
+// workgroup (store_partials) and a finisher that sums the slots in order and
+// applies the scalar update of the reference sequence it replaces. The
+// finisher is the row kernel's own last workgroup (last_workgroup) or, where
+// that is slower, a launch of one workgroup.
+
+// Finishers: the FP64 total of `count` partials as a normalized pair, then the
+// reference's scalar kernel on it.
+enum class Finish { Alpha, Check, Beta, Pair, BicgBeta, BicgAlpha, BicgS };
+template <Finish F, bool kHere = false>
+__device__ __forceinline__ void finish_body(const double* __restrict__ partials, unsigned count,
+                                            float* scalars, int* status, float* dst) {
+  if (status[0] != 0) return;
+  double total[1];
+  sum_partials<1, kHere>(partials, count, total);
+  if (threadIdx.x != 0) return;
+  const Pair value = to_pair(total[0]);
+  if constexpr (F == Finish::Alpha) {
+    pstore(scalars, 2, value);
+    pcg_alpha(scalars, status);
+  } else if constexpr (F == Finish::Check) {
+    pstore(scalars, 18, value);
+    solver_check_body(scalars, status, 1);
+  } else if constexpr (F == Finish::Beta) {
+    pstore(scalars, 4, value);
+    pcg_beta(scalars, status, 0);
+  } else if constexpr (F == Finish::BicgBeta) {
+    pstore(scalars, 0, value);
+    bicg_beta(scalars, status);
+  } else if constexpr (F == Finish::BicgAlpha) {
+    pstore(scalars, 2, value);
+    bicg_alpha(scalars, status);
+  } else if constexpr (F == Finish::BicgS) {
+    pstore(scalars, 16, value);
+    bicg_s(scalars, status);
+  } else {
+    pstore(dst, 0, value);
+  }
+}
+// Two-slot finishers. Omega: t.t, t.s into slots 2 and 4, then bicg_omega.
+// CheckBeta: r.r into slot 18 and the check (which keeps slot 0 as the
+// previous rho in slot 14), then, if the iteration goes on, shadow.r into
+// slot 0 and the next iteration's bicg_beta.
+enum class Finish2 { Omega, CheckBeta };
+template <Finish2 F, bool kHere = false>
+__device__ __forceinline__ void finish2_body(const double* __restrict__ partials, unsigned count,
+                                             float* scalars, int* status) {
+  if (status[0] != 0) return;
+  double total[2];
+  sum_partials<2, kHere>(partials, count, total);
+  if (threadIdx.x != 0) return;
+  if constexpr (F == Finish2::Omega) {
+    pstore(scalars, 2, to_pair(total[0]));
+    pstore(scalars, 4, to_pair(total[1]));
+    bicg_omega(scalars, status);
+  } else {
+    pstore(scalars, 18, to_pair(total[0]));
+    solver_check_body(scalars, status, 0);
+    if (status[0] != 0) return;
+    pstore(scalars, 0, to_pair(total[1]));
+    bicg_beta(scalars, status);
+  }
+}
+// How a row kernel ends its reduction: in its last workgroup if it has
+// tickets, else in a launch that follows.
+struct Ending {
+  unsigned* tickets = nullptr;
+  float* scalars = nullptr;
+  int* status = nullptr;
+  float* dst = nullptr;
+};
+template <Finish F>
+__device__ __forceinline__ void end_reduction(const double (&mine)[1], double* partials, const Ending& e) {
+  if (e.tickets == nullptr) store_partials<1>(mine, partials);
+  else if (last_workgroup<1>(mine, partials, e.tickets))
+    finish_body<F, true>(partials, gridDim.x, e.scalars, e.status, e.dst);
+}
+template <Finish2 F>
+__device__ __forceinline__ void end_reduction(const double (&mine)[2], double* partials, const Ending& e) {
+  if (e.tickets == nullptr) store_partials<2>(mine, partials);
+  else if (last_workgroup<2>(mine, partials, e.tickets))
+    finish2_body<F, true>(partials, gridDim.x, e.scalars, e.status);
+}
 
 // q = A p, partials of p.q: csr_spmv_guarded + dot_into(p,q,2).
 __global__ void __launch_bounds__(kBlock) k_fused_spmv_dot(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ p,
-    float* __restrict__ q, const int* __restrict__ status, double* __restrict__ partials) {
+    float* __restrict__ q, const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -524,12 +604,12 @@ __global__ void __launch_bounds__(kBlock) k_fused_spmv_dot(int n, const int* __r
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::Alpha>(mine, partials, ending);
 }
 // x += alpha p, r -= alpha q, partials of r.r: solver_step + dot_into(r,r,18).
 __global__ void __launch_bounds__(kBlock) k_fused_step_dot(int n, float* __restrict__ x,
     float* __restrict__ r, const float* __restrict__ p, const float* __restrict__ q,
-    const float* __restrict__ scalars, const int* __restrict__ status, double* __restrict__ partials) {
+    const float* scalars, const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   const float alpha = pfloat(pload(scalars, 8));
@@ -542,14 +622,14 @@ __global__ void __launch_bounds__(kBlock) k_fused_step_dot(int n, float* __restr
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::Check>(mine, partials, ending);
 }
 // Final smoothing sweep of the preconditioner, partials of r.z:
 // amg_smooth + dot_into(r,z,4). Here b is the Krylov residual r.
 __global__ void __launch_bounds__(kBlock) k_fused_smooth_dot(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ x,
     const float* __restrict__ b, const float* __restrict__ inverse, float* __restrict__ next,
-    const int* __restrict__ status, double* __restrict__ partials) {
+    const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -562,14 +642,14 @@ __global__ void __launch_bounds__(kBlock) k_fused_smooth_dot(int n, const int* _
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::Beta>(mine, partials, ending);
 }
 // Smoothing sweep whose output is summed for the constant-nullspace
 // projection that follows: amg_smooth + sum_into(next).
 __global__ void __launch_bounds__(kBlock) k_fused_smooth_partial_sum(int n,
     const int* __restrict__ rows, const int* __restrict__ cols, const float* __restrict__ values,
     const float* __restrict__ x, const float* __restrict__ b, const float* __restrict__ inverse,
-    float* __restrict__ next, const int* __restrict__ status, double* __restrict__ partials) {
+    float* __restrict__ next, const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -581,12 +661,12 @@ __global__ void __launch_bounds__(kBlock) k_fused_smooth_partial_sum(int n,
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::Pair>(mine, partials, ending);
 }
 // Mean removal, partials of r.z: solver_project + dot_into(r,z,4).
 __global__ void __launch_bounds__(kBlock) k_fused_project_dot(int n, float* __restrict__ z,
     const float* __restrict__ sum, float count_hi, float count_lo, const float* __restrict__ r,
-    const int* __restrict__ status, double* __restrict__ partials) {
+    const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -597,7 +677,7 @@ __global__ void __launch_bounds__(kBlock) k_fused_project_dot(int n, float* __re
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::Beta>(mine, partials, ending);
 }
 
 // BiCGStab with the Jacobi preconditioner (linalg/solver.cpp:314-361). Each
@@ -608,13 +688,13 @@ __global__ void __launch_bounds__(kBlock) k_fused_project_dot(int n, float* __re
 
 // Partials of x.y: dot_into(x, y) ahead of a scalar update.
 __device__ __forceinline__ void fused_dot_body(int n, const float* __restrict__ x,
-    const float* __restrict__ y, const int* __restrict__ status, double* __restrict__ partials) {
+    const float* __restrict__ y, const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {i < n ? double(x[i]) * double(y[i]) : 0.0};
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::BicgBeta>(mine, partials, ending);
 }
 // p = r + beta (p - omega q), z = p * inverse: solver_bicg_direction +
 // krylov_multiply_guarded.
@@ -632,8 +712,8 @@ __device__ __forceinline__ void fused_bicg_direction_body(int n, const float* __
 // q = A z, partials of shadow.q: csr_spmv_guarded + dot_into(shadow, q, 2).
 __device__ __forceinline__ void fused_spmv_shadow_dot_body(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ z,
-    float* __restrict__ q, const float* __restrict__ shadow, const int* __restrict__ status,
-    double* __restrict__ partials) {
+    float* __restrict__ q, const float* __restrict__ shadow, const int* status,
+    double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -644,14 +724,14 @@ __device__ __forceinline__ void fused_spmv_shadow_dot_body(int n, const int* __r
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::BicgAlpha>(mine, partials, ending);
 }
 // s = r - alpha q, zs = s * inverse, partials of s.s: solver_bicg_difference +
 // dot_into(s, s, 16) + krylov_multiply_guarded.
 __device__ __forceinline__ void fused_bicg_difference_body(int n, const float* __restrict__ r,
     const float* __restrict__ q, float* __restrict__ sv, const float* __restrict__ inverse,
-    float* __restrict__ zs, const float* __restrict__ scalars, const int* __restrict__ status,
-    double* __restrict__ partials) {
+    float* __restrict__ zs, const float* scalars, const int* status,
+    double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[1] = {0.0};
@@ -663,13 +743,13 @@ __device__ __forceinline__ void fused_bicg_difference_body(int n, const float* _
   }
   __shared__ double lds[kBlock / 64];
   mine[0] = block_sum(mine[0], lds);
-  store_partials<1>(mine, partials);
+  end_reduction<Finish::BicgS>(mine, partials, ending);
 }
 // t = A zs, partials of t.t and t.s: csr_spmv_guarded + dot2_into(t,t,t,s,2).
 __device__ __forceinline__ void fused_spmv_dot2_body(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ zs,
-    float* __restrict__ t, const float* __restrict__ sv, const int* __restrict__ status,
-    double* __restrict__ partials) {
+    float* __restrict__ t, const float* __restrict__ sv, const int* status,
+    double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[2] = {0.0, 0.0};
@@ -682,7 +762,7 @@ __device__ __forceinline__ void fused_spmv_dot2_body(int n, const int* __restric
   __shared__ double lds[2][kBlock / 64];
   mine[0] = block_sum(mine[0], lds[0]);
   mine[1] = block_sum(mine[1], lds[1]);
-  store_partials<2>(mine, partials);
+  end_reduction<Finish2::Omega>(mine, partials, ending);
 }
 // x += alpha z + omega zs, r = s - omega t (or the s exit), partials of r.r
 // and shadow.r: solver_bicg_step + dot_into(r, r, 18) + the next
@@ -690,7 +770,7 @@ __device__ __forceinline__ void fused_spmv_dot2_body(int n, const int* __restric
 __device__ __forceinline__ void fused_bicg_step_body(int n, float* __restrict__ x,
     float* __restrict__ r, const float* __restrict__ z, const float* __restrict__ zs,
     const float* __restrict__ sv, const float* __restrict__ t, const float* __restrict__ shadow,
-    const float* __restrict__ scalars, const int* __restrict__ status, double* __restrict__ partials) {
+    const float* scalars, const int* status, double* partials, Ending ending) {
   if (status[0] != 0) return;
   const int i = row_index();
   double mine[2] = {0.0, 0.0};
@@ -711,13 +791,13 @@ __device__ __forceinline__ void fused_bicg_step_body(int n, float* __restrict__ 
   __shared__ double lds[2][kBlock / 64];
   mine[0] = block_sum(mine[0], lds[0]);
   mine[1] = block_sum(mine[1], lds[1]);
-  store_partials<2>(mine, partials);
+  end_reduction<Finish2::CheckBeta>(mine, partials, ending);
 }
 
 // Single-system kernels (one BiCGStab solve per launch).
 __global__ void __launch_bounds__(kBlock) k_fused_dot(int n, const float* __restrict__ x,
-    const float* __restrict__ y, const int* __restrict__ status, double* __restrict__ partials) {
-  fused_dot_body(n, x, y, status, partials);
+    const float* __restrict__ y, const int* status, double* partials, Ending ending) {
+  fused_dot_body(n, x, y, status, partials, ending);
 }
 __global__ void __launch_bounds__(kBlock) k_fused_bicg_direction(int n, const float* __restrict__ r,
     const float* __restrict__ q, float* __restrict__ p, const float* __restrict__ inverse,
@@ -726,27 +806,27 @@ __global__ void __launch_bounds__(kBlock) k_fused_bicg_direction(int n, const fl
 }
 __global__ void __launch_bounds__(kBlock) k_fused_spmv_shadow_dot(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ z,
-    float* __restrict__ q, const float* __restrict__ shadow, const int* __restrict__ status,
-    double* __restrict__ partials) {
-  fused_spmv_shadow_dot_body(n, rows, cols, values, z, q, shadow, status, partials);
+    float* __restrict__ q, const float* __restrict__ shadow, const int* status,
+    double* partials, Ending ending) {
+  fused_spmv_shadow_dot_body(n, rows, cols, values, z, q, shadow, status, partials, ending);
 }
 __global__ void __launch_bounds__(kBlock) k_fused_bicg_difference(int n, const float* __restrict__ r,
     const float* __restrict__ q, float* __restrict__ sv, const float* __restrict__ inverse,
-    float* __restrict__ zs, const float* __restrict__ scalars, const int* __restrict__ status,
-    double* __restrict__ partials) {
-  fused_bicg_difference_body(n, r, q, sv, inverse, zs, scalars, status, partials);
+    float* __restrict__ zs, const float* scalars, const int* status,
+    double* partials, Ending ending) {
+  fused_bicg_difference_body(n, r, q, sv, inverse, zs, scalars, status, partials, ending);
 }
 __global__ void __launch_bounds__(kBlock) k_fused_spmv_dot2(int n, const int* __restrict__ rows,
     const int* __restrict__ cols, const float* __restrict__ values, const float* __restrict__ zs,
-    float* __restrict__ t, const float* __restrict__ sv, const int* __restrict__ status,
-    double* __restrict__ partials) {
-  fused_spmv_dot2_body(n, rows, cols, values, zs, t, sv, status, partials);
+    float* __restrict__ t, const float* __restrict__ sv, const int* status,
+    double* partials, Ending ending) {
+  fused_spmv_dot2_body(n, rows, cols, values, zs, t, sv, status, partials, ending);
 }
 __global__ void __launch_bounds__(kBlock) k_fused_bicg_step(int n, float* __restrict__ x,
     float* __restrict__ r, const float* __restrict__ z, const float* __restrict__ zs,
     const float* __restrict__ sv, const float* __restrict__ t, const float* __restrict__ shadow,
-    const float* __restrict__ scalars, const int* __restrict__ status, double* __restrict__ partials) {
-  fused_bicg_step_body(n, x, r, z, zs, sv, t, shadow, scalars, status, partials);
+    const float* scalars, const int* status, double* partials, Ending ending) {
+  fused_bicg_step_body(n, x, r, z, zs, sv, t, shadow, scalars, status, partials, ending);
 }
 
 // Batched kernels (no reference counterpart): lane blockIdx.y of a
@@ -759,6 +839,9 @@ __global__ void __launch_bounds__(kBlock) k_fused_bicg_step(int n, float* __rest
   if (((mask >> lane) & 1) == 0) return;                \
   const kh_bicg_lane& L = lanes[lane];                  \
   double* part = partials + std::size_t(lane) * stride;
+__device__ __forceinline__ Ending lane_ending(const kh_bicg_lane& L, int lane, unsigned* tickets) {
+  return {tickets != nullptr ? tickets + lane * kTicketWords : nullptr, L.scalars, L.status, nullptr};
+}
 __global__ void __launch_bounds__(kBlock) k_batch_bicg_direction(int n, const kh_bicg_lane* __restrict__ lanes,
                                                                  int mask, double* partials, unsigned stride) {
   LANE_OR_RETURN
@@ -766,24 +849,24 @@ __global__ void __launch_bounds__(kBlock) k_batch_bicg_direction(int n, const kh
   fused_bicg_direction_body(n, L.r, L.q, L.p, L.inverse, L.z, L.scalars, L.status);
 }
 __global__ void __launch_bounds__(kBlock) k_batch_spmv_shadow_dot(int n, const kh_bicg_lane* __restrict__ lanes,
-                                                                  int mask, double* partials, unsigned stride) {
+                                                                  int mask, double* partials, unsigned stride, unsigned* tickets) {
   LANE_OR_RETURN
-  fused_spmv_shadow_dot_body(n, L.row_ptr, L.col, L.val, L.z, L.q, L.shadow, L.status, part);
+  fused_spmv_shadow_dot_body(n, L.row_ptr, L.col, L.val, L.z, L.q, L.shadow, L.status, part, lane_ending(L, lane, tickets));
 }
 __global__ void __launch_bounds__(kBlock) k_batch_bicg_difference(int n, const kh_bicg_lane* __restrict__ lanes,
-                                                                  int mask, double* partials, unsigned stride) {
+                                                                  int mask, double* partials, unsigned stride, unsigned* tickets) {
   LANE_OR_RETURN
-  fused_bicg_difference_body(n, L.r, L.q, L.s, L.inverse, L.zs, L.scalars, L.status, part);
+  fused_bicg_difference_body(n, L.r, L.q, L.s, L.inverse, L.zs, L.scalars, L.status, part, lane_ending(L, lane, tickets));
 }
 __global__ void __launch_bounds__(kBlock) k_batch_spmv_dot2(int n, const kh_bicg_lane* __restrict__ lanes,
-                                                            int mask, double* partials, unsigned stride) {
+                                                            int mask, double* partials, unsigned stride, unsigned* tickets) {
   LANE_OR_RETURN
-  fused_spmv_dot2_body(n, L.row_ptr, L.col, L.val, L.zs, L.t, L.s, L.status, part);
+  fused_spmv_dot2_body(n, L.row_ptr, L.col, L.val, L.zs, L.t, L.s, L.status, part, lane_ending(L, lane, tickets));
 }
 __global__ void __launch_bounds__(kBlock) k_batch_bicg_step(int n, const kh_bicg_lane* __restrict__ lanes,
-                                                            int mask, double* partials, unsigned stride) {
+                                                            int mask, double* partials, unsigned stride, unsigned* tickets) {
   LANE_OR_RETURN
-  fused_bicg_step_body(n, L.x, L.r, L.z, L.zs, L.s, L.t, L.shadow, L.scalars, L.status, part);
+  fused_bicg_step_body(n, L.x, L.r, L.z, L.zs, L.s, L.t, L.shadow, L.scalars, L.status, part, lane_ending(L, lane, tickets));
 }
 
 // The K-cycle's inner corrections in four fused steps (no reference
@@ -895,63 +978,6 @@ __global__ void __launch_bounds__(kBlock) k_inner_finish(const double* __restric
   }
 }
 
-// Finishers: the FP64 total of `count` partials as a normalized pair, then the
-// reference's scalar kernel on it.
-enum class Finish { Alpha, Check, Beta, Pair, BicgBeta, BicgAlpha, BicgS };
-template <Finish F>
-__device__ __forceinline__ void finish_body(const double* __restrict__ partials, unsigned count,
-                                            float* scalars, int* status, float* dst) {
-  if (status[0] != 0) return;
-  double total[1];
-  sum_partials<1>(partials, count, total);
-  if (threadIdx.x != 0) return;
-  const Pair value = to_pair(total[0]);
-  if constexpr (F == Finish::Alpha) {
-    pstore(scalars, 2, value);
-    pcg_alpha(scalars, status);
-  } else if constexpr (F == Finish::Check) {
-    pstore(scalars, 18, value);
-    solver_check_body(scalars, status, 1);
-  } else if constexpr (F == Finish::Beta) {
-    pstore(scalars, 4, value);
-    pcg_beta(scalars, status, 0);
-  } else if constexpr (F == Finish::BicgBeta) {
-    pstore(scalars, 0, value);
-    bicg_beta(scalars, status);
-  } else if constexpr (F == Finish::BicgAlpha) {
-    pstore(scalars, 2, value);
-    bicg_alpha(scalars, status);
-  } else if constexpr (F == Finish::BicgS) {
-    pstore(scalars, 16, value);
-    bicg_s(scalars, status);
-  } else {
-    pstore(dst, 0, value);
-  }
-}
-// Two-slot finishers. Omega: t.t, t.s into slots 2 and 4, then bicg_omega.
-// CheckBeta: r.r into slot 18 and the check (which keeps slot 0 as the
-// previous rho in slot 14), then, if the iteration goes on, shadow.r into
-// slot 0 and the next iteration's bicg_beta.
-enum class Finish2 { Omega, CheckBeta };
-template <Finish2 F>
-__device__ __forceinline__ void finish2_body(const double* __restrict__ partials, unsigned count,
-                                             float* scalars, int* status) {
-  if (status[0] != 0) return;
-  double total[2];
-  sum_partials<2>(partials, count, total);
-  if (threadIdx.x != 0) return;
-  if constexpr (F == Finish2::Omega) {
-    pstore(scalars, 2, to_pair(total[0]));
-    pstore(scalars, 4, to_pair(total[1]));
-    bicg_omega(scalars, status);
-  } else {
-    pstore(scalars, 18, to_pair(total[0]));
-    solver_check_body(scalars, status, 0);
-    if (status[0] != 0) return;
-    pstore(scalars, 0, to_pair(total[1]));
-    bicg_beta(scalars, status);
-  }
-}
 template <Finish F>
 __global__ void __launch_bounds__(kBlock) k_finish(const double* __restrict__ partials,
                                                    unsigned count, float* scalars, int* status,
@@ -1606,12 +1632,23 @@ unsigned reduce_grid(int n) {
     throw std::runtime_error("fused reduction kernel: n exceeds 16,777,216 rows");
   return blocks;
 }
+// The tickets of a reduction over g workgroups, or null where a launch of its
+// own finishes it. The last workgroup saves a launch of some 3.5 us (and the
+// gap before it) but the ticket counters take a time of their own: with all
+// reductions finished that way against none, batched BiCGStab iterations of
+// 594 workgroups a lane went from 51.8 to 47.3 us, SIMPLEC iterations of 4
+// workgroups from 3.14 to 2.90 ms; of 2000 workgroups they took 4.5 ms
+// against 4.3 with launches above this line, and a solve of 3900 workgroups
+// 17.8 ms against 17.5.
+constexpr unsigned kTicketBlocks = 1024;
+unsigned* tickets(kh_device* d, unsigned g) { return g <= kTicketBlocks ? d->tickets : nullptr; }
 #define FINISH dim3(1), dim3(kBlock), 0, d->stream
 void l_fused_spmv_dot_alpha(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 6));
-  k_fused_spmv_dot<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), st, d->partials);
-  k_finish<Finish::Alpha><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
+  const Ending ending{tickets(d, g), KF(5), st, nullptr};
+  k_fused_spmv_dot<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::Alpha><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
 }
 void l_inner_first_step(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
@@ -1642,8 +1679,9 @@ void l_inner_second_step(kh_device* d, int n, const kh_arg* a) {
 void l_fused_step_dot_check(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 5));
-  k_fused_step_dot<<<GRID(n)>>>(n, KF(0), KF(1), KCF(2), KCF(3), KCF(4), st, d->partials);
-  k_finish<Finish::Check><<<FINISH>>>(d->partials, g, KF(4), st, nullptr);
+  const Ending ending{tickets(d, g), KF(4), st, nullptr};
+  k_fused_step_dot<<<GRID(n)>>>(n, KF(0), KF(1), KCF(2), KCF(3), KCF(4), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::Check><<<FINISH>>>(d->partials, g, KF(4), st, nullptr);
 }
 void l_fused_residual_restrict(kh_device* d, int n, const kh_arg* a) {
   const unsigned groups = unsigned((n + kRestrictRows - 1) / kRestrictRows);
@@ -1687,16 +1725,18 @@ void l_fused_prolong_smooth(kh_device* d, int n, const kh_arg* a) {
 void l_fused_smooth_dot_beta(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 7));
+  const Ending ending{tickets(d, g), KF(8), st, nullptr};
   k_fused_smooth_dot<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KCF(4), KCF(5), KF(6), st,
-                                  d->partials);
-  k_finish<Finish::Beta><<<FINISH>>>(d->partials, g, KF(8), st, nullptr);
+                                  d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::Beta><<<FINISH>>>(d->partials, g, KF(8), st, nullptr);
 }
 void l_fused_smooth_sum(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = const_cast<int*>(KB(7));
+  const Ending ending{tickets(d, g), nullptr, st, KF(8)};
   k_fused_smooth_partial_sum<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KCF(4), KCF(5), KF(6),
-                                          st, d->partials);
-  k_finish<Finish::Pair><<<FINISH>>>(d->partials, g, nullptr, st, KF(8));
+                                          st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::Pair><<<FINISH>>>(d->partials, g, nullptr, st, KF(8));
 }
 void l_fused_smooth_from_zero(kh_device* d, int n, const kh_arg* a) {
   k_fused_smooth_from_zero<float><<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KCF(4), KF(5), KB(6));
@@ -1736,8 +1776,9 @@ void l_fused_coarse_tail(kh_device* d, int n, const kh_arg* a) {
 void l_fused_dot_bicg_beta(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 3));
-  k_fused_dot<<<GRID(n)>>>(n, KCF(0), KCF(1), st, d->partials);
-  k_finish<Finish::BicgBeta><<<FINISH>>>(d->partials, g, KF(2), st, nullptr);
+  const Ending ending{tickets(d, g), KF(2), st, nullptr};
+  k_fused_dot<<<GRID(n)>>>(n, KCF(0), KCF(1), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::BicgBeta><<<FINISH>>>(d->partials, g, KF(2), st, nullptr);
 }
 void l_fused_bicg_direction(kh_device* d, int n, const kh_arg* a) {
   k_fused_bicg_direction<<<GRID(n)>>>(n, KCF(0), KCF(1), KF(2), KCF(3), KF(4), KCF(5), KB(6));
@@ -1745,27 +1786,31 @@ void l_fused_bicg_direction(kh_device* d, int n, const kh_arg* a) {
 void l_fused_spmv_shadow_alpha(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 7));
-  k_fused_spmv_shadow_dot<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), KCF(5), st, d->partials);
-  k_finish<Finish::BicgAlpha><<<FINISH>>>(d->partials, g, KF(6), st, nullptr);
+  const Ending ending{tickets(d, g), KF(6), st, nullptr};
+  k_fused_spmv_shadow_dot<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), KCF(5), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::BicgAlpha><<<FINISH>>>(d->partials, g, KF(6), st, nullptr);
 }
 void l_fused_bicg_difference_s(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 6));
-  k_fused_bicg_difference<<<GRID(n)>>>(n, KCF(0), KCF(1), KF(2), KCF(3), KF(4), KCF(5), st, d->partials);
-  k_finish<Finish::BicgS><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
+  const Ending ending{tickets(d, g), KF(5), st, nullptr};
+  k_fused_bicg_difference<<<GRID(n)>>>(n, KCF(0), KCF(1), KF(2), KCF(3), KF(4), KCF(5), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::BicgS><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
 }
 void l_fused_spmv_dot2_omega(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 7));
-  k_fused_spmv_dot2<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), KCF(5), st, d->partials);
-  k_finish2<Finish2::Omega><<<FINISH>>>(d->partials, g, KF(6), st);
+  const Ending ending{tickets(d, g), KF(6), st, nullptr};
+  k_fused_spmv_dot2<<<GRID(n)>>>(n, KB(0), KB(1), KCF(2), KCF(3), KF(4), KCF(5), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish2<Finish2::Omega><<<FINISH>>>(d->partials, g, KF(6), st);
 }
 void l_fused_bicg_step_check_beta(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 8));
+  const Ending ending{tickets(d, g), KF(7), st, nullptr};
   k_fused_bicg_step<<<GRID(n)>>>(n, KF(0), KF(1), KCF(2), KCF(3), KCF(4), KCF(5), KCF(6), KCF(7), st,
-                                 d->partials);
-  k_finish2<Finish2::CheckBeta><<<FINISH>>>(d->partials, g, KF(7), st);
+                                 d->partials, ending);
+  if (ending.tickets == nullptr) k_finish2<Finish2::CheckBeta><<<FINISH>>>(d->partials, g, KF(7), st);
 }
 // Batched BiCGStab-Jacobi launches: n = rows of every lane; lanes (device
 // array of kh_bicg_lane), lane count (1..KH_BATCH_MAX_LANES), mask of the
@@ -1789,35 +1834,40 @@ void l_batch_spmv_shadow_alpha(kh_device* d, int n, const kh_arg* a) {
   const int count = i32(a, 1), mask = i32(a, 2);
   const unsigned stride = batch_stride(n, count), g = reduce_grid(n);
   const auto* lanes = static_cast<const kh_bicg_lane*>(buf(a, 0));
-  k_batch_spmv_shadow_dot<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride);
-  k_batch_finish<Finish::BicgAlpha><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
+  unsigned* const t = tickets(d, g);
+  k_batch_spmv_shadow_dot<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride, t);
+  if (t == nullptr) k_batch_finish<Finish::BicgAlpha><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
 }
 void l_batch_bicg_difference_s(kh_device* d, int n, const kh_arg* a) {
   const int count = i32(a, 1), mask = i32(a, 2);
   const unsigned stride = batch_stride(n, count), g = reduce_grid(n);
   const auto* lanes = static_cast<const kh_bicg_lane*>(buf(a, 0));
-  k_batch_bicg_difference<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride);
-  k_batch_finish<Finish::BicgS><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
+  unsigned* const t = tickets(d, g);
+  k_batch_bicg_difference<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride, t);
+  if (t == nullptr) k_batch_finish<Finish::BicgS><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
 }
 void l_batch_spmv_dot2_omega(kh_device* d, int n, const kh_arg* a) {
   const int count = i32(a, 1), mask = i32(a, 2);
   const unsigned stride = batch_stride(n, count), g = reduce_grid(n);
   const auto* lanes = static_cast<const kh_bicg_lane*>(buf(a, 0));
-  k_batch_spmv_dot2<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride);
-  k_batch_finish2<Finish2::Omega><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
+  unsigned* const t = tickets(d, g);
+  k_batch_spmv_dot2<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride, t);
+  if (t == nullptr) k_batch_finish2<Finish2::Omega><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
 }
 void l_batch_bicg_step_check_beta(kh_device* d, int n, const kh_arg* a) {
   const int count = i32(a, 1), mask = i32(a, 2);
   const unsigned stride = batch_stride(n, count), g = reduce_grid(n);
   const auto* lanes = static_cast<const kh_bicg_lane*>(buf(a, 0));
-  k_batch_bicg_step<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride);
-  k_batch_finish2<Finish2::CheckBeta><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
+  unsigned* const t = tickets(d, g);
+  k_batch_bicg_step<<<BATCH_GRID(n, count)>>>(n, lanes, mask, d->partials, stride, t);
+  if (t == nullptr) k_batch_finish2<Finish2::CheckBeta><<<BATCH_FINISH(count)>>>(lanes, mask, d->partials, stride, g);
 }
 void l_fused_project_dot_beta(kh_device* d, int n, const kh_arg* a) {
   const unsigned g = reduce_grid(n);
   int* st = static_cast<int*>(buf(a, 6));
-  k_fused_project_dot<<<GRID(n)>>>(n, KF(0), KCF(1), f32(a, 2), f32(a, 3), KCF(4), st, d->partials);
-  k_finish<Finish::Beta><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
+  const Ending ending{tickets(d, g), KF(5), st, nullptr};
+  k_fused_project_dot<<<GRID(n)>>>(n, KF(0), KCF(1), f32(a, 2), f32(a, 3), KCF(4), st, d->partials, ending);
+  if (ending.tickets == nullptr) k_finish<Finish::Beta><<<FINISH>>>(d->partials, g, KF(5), st, nullptr);
 }
 
 }  // namespace

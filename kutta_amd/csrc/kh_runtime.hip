@@ -262,6 +262,8 @@ int kh_create(int ordinal, kh_device** out) {
       d->name += (d->name.empty() ? "" : " ") + std::string(prop.gcnArchName);
     check(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking), "hipStreamCreate");
     check(hipMalloc(&d->partials, sizeof(double) * 2 * kMaxReduceBlocks), "hipMalloc partials");
+    check(hipMalloc(&d->tickets, sizeof(unsigned) * kTicketWords * KH_BATCH_MAX_LANES), "hipMalloc tickets");
+    check(hipMemset(d->tickets, 0, sizeof(unsigned) * kTicketWords * KH_BATCH_MAX_LANES), "hipMemset tickets");
     check(hipMalloc(&d->results, sizeof(double) * kMaxHostResults), "hipMalloc results");
     check(hipHostMalloc(&d->results_host, sizeof(double) * kMaxHostResults, hipHostMallocDefault),
           "hipHostMalloc results");
@@ -282,6 +284,7 @@ void kh_destroy(kh_device* d) {
     }
   for (auto e : d->event_pool) (void)hipEventDestroy(e);
   (void)hipFree(d->partials);
+  (void)hipFree(d->tickets);
   (void)hipFree(d->results);
   (void)hipHostFree(d->results_host);
   (void)hipStreamDestroy(d->stream);
