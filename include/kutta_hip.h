@@ -509,7 +509,7 @@ typedef struct kh_grid_part {
 /* Chunks a row of `chunks` takes: an odd number when long, so that the rows of
  * neighbouring lanes start on different LDS banks. */
 #define KH_GRID_CHUNKS(chunks) ((chunks) > 3 ? (chunks) | 1 : (chunks))
-#define KH_GRID_CTL_WORDS 128
+#define KH_GRID_CTL_WORDS 160
 #define KH_GRID_POOL_WORDS 39936
 
 /* Device::launch (device.hpp:205; cuda_device.cu:132-140): runs kernel `kernel`

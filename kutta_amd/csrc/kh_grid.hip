@@ -29,6 +29,7 @@
 // waits for one that may not be running: the barrier is used only after all
 // have met.
 #include "kh_device_math.hpp"
+#include "kh_grid_gather.hpp"
 
 namespace kh {
 namespace {
@@ -36,19 +37,6 @@ namespace {
 constexpr int kGridThreads = 1024;
 constexpr int kCoarseMax = 24;  // largest coarsest level solved by amg_coarse_solve (linalg/amg.cpp:287)
 constexpr int kMaxLevels = 16;
-
-// Control block (KH_GRID_CTL_WORDS words, in cache lines of their own).
-// `count` packs three 16-bit counters: workgroups started, ranks taken,
-// workgroups done; the last one done clears the block for the next launch.
-struct GridCtl {
-  unsigned long long* count;
-  unsigned* state;  // 0 gathering, 1 all met, 2 one workgroup works alone
-  unsigned* bar;
-  unsigned* home;
-  __device__ explicit GridCtl(unsigned* w)
-      : count(reinterpret_cast<unsigned long long*>(w)), state(w + 32), bar(w + 64), home(w + 96) {}
-};
-constexpr unsigned long long kRankOne = 1ull << 16, kDoneOne = 1ull << 32;
 
 __device__ __forceinline__ unsigned xcc_id() {
   unsigned v;
@@ -72,64 +60,36 @@ __device__ __forceinline__ unsigned ctl_load(const unsigned* p) {
 // Every earlier store of this wavefront has reached the coherence point.
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-enum class GridRole { Leave, Member, Solo };
-struct GridPlace {
-  GridRole role;
-  int rank;
+// Control block (KH_GRID_CTL_WORDS words, in cache lines of their own), as
+// kh_grid_gather.hpp uses it; the limit is in ticks of the 100 MHz clock.
+struct GridCtl {
+  unsigned *arrived, *settled, *bar, *home, *left;
+  long limit;
+  long long start = 0;
+  __device__ GridCtl(unsigned* w, long limit_ticks)
+      : arrived(w), settled(w + 32), bar(w + 64), home(w + 96), left(w + 128), limit(limit_ticks) {}
+  __device__ static unsigned add(unsigned* p, unsigned v) {
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ unsigned arrive(unsigned v) { return add(arrived, v); }
+  __device__ unsigned arrivals() { return ctl_load(arrived); }
+  __device__ unsigned settle(unsigned to) {
+    unsigned expected = 0;
+    __hip_atomic_compare_exchange_strong(settled, &expected, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    stores_done();  // also where the result is not used
+    return expected;
+  }
+  __device__ unsigned state() { return ctl_load(settled); }
+  __device__ unsigned leave() { return add(left, 1); }
+  __device__ void wait() { start = wall_clock64(); }
+  __device__ bool expired() { return wall_clock64() - start > limit; }
+  __device__ void clear() {
+    for (unsigned* p : {bar, left, settled, arrived})
+      __hip_atomic_store(p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 };
 
-__device__ __forceinline__ void grid_clear(const GridCtl& c) {
-  __hip_atomic_store(c.bar, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(c.state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(c.count, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned grid_settle(const GridCtl& c, unsigned to) {
-  unsigned expected = 0;
-  __hip_atomic_compare_exchange_strong(c.state, &expected, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-  return expected;  // 0: this call settled it
-}
-// Thread 0 of a workgroup enters; a workgroup that is to leave has left.
-// `limit` is the longest wait for the others in ticks of the 100 MHz clock.
-__device__ GridPlace grid_enter(const GridCtl& c, int parts, long limit) {
-  const unsigned grid = gridDim.x;
-  const bool here = xcc_id() == ctl_load(c.home);
-  const unsigned long long old = __hip_atomic_fetch_add(
-      c.count, here ? 1ull + kRankOne : 1ull + kDoneOne, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned started = unsigned(old & 0xffff) + 1, rank = unsigned(old >> 16) & 0xffff;
-  const bool last = started == grid;
-  if (!here) {
-    // The last to start speaks for all; if no workgroup is on the home XCD it
-    // works alone.
-    if (last && rank == 0) {
-      grid_settle(c, 2);
-      __hip_atomic_fetch_add(c.count, 0ull - kDoneOne, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return {GridRole::Solo, 0};
-    }
-    if (last) grid_settle(c, 1);
-    if (unsigned(old >> 32) + 1 == grid) grid_clear(c);
-    return {GridRole::Leave, 0};
-  }
-  if (last) grid_settle(c, 1);
-  unsigned state;
-  const long long start = wall_clock64();
-  while ((state = ctl_load(c.state)) == 0) {
-    if (wall_clock64() - start > limit && grid_settle(c, 2) == 0) return {GridRole::Solo, int(rank)};
-  }
-  if (state == 1) {
-    const unsigned long long met =
-        __hip_atomic_load(c.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 16 & 0xffff;
-    if (int(met) == parts) return {GridRole::Member, int(rank)};
-    if (rank == 0) return {GridRole::Solo, 0};
-  }
-  return {GridRole::Leave, -1};
-}
-// Thread 0 of a workgroup that took a rank (or works alone) leaves.
-__device__ __forceinline__ void grid_leave(const GridCtl& c) {
-  const unsigned long long old =
-      __hip_atomic_fetch_add(c.count, kDoneOne, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (unsigned(old >> 32) + 1 == gridDim.x) grid_clear(c);
-}
 // Barrier over the members: all of them are running (grid_enter), and each
 // passes the same barriers, so the wait ends; it is bounded all the same.
 constexpr unsigned kBarrierSpins = 1u << 21;  // of some 0.3 us each
@@ -537,14 +497,14 @@ __device__ __forceinline__ void member_cycle(const CycleArgs& A, const GridCtl& 
 __global__ void __launch_bounds__(kGridThreads) k_grid_cycle(const CycleArgs A) {
   if (A.status[0] != 0) return;
   __shared__ GridPlace place;
-  const GridCtl ctl(A.ctl);
-  if (threadIdx.x == 0) place = grid_enter(ctl, A.parts, long(A.limit_us) * 100);
+  GridCtl ctl(A.ctl, long(A.limit_us) * 100);
+  if (threadIdx.x == 0) place = grid_enter(ctl, gridDim.x, A.parts, xcc_id() == ctl_load(ctl.home));
   __syncthreads();
   const GridRole role = GridRole(__builtin_amdgcn_readfirstlane(int(place.role)));
   if (role == GridRole::Member) member_cycle(A, ctl, __builtin_amdgcn_readfirstlane(place.rank));
   else if (role == GridRole::Solo) solo_cycle(A);
   __syncthreads();
-  if (threadIdx.x == 0 && (role != GridRole::Leave || place.rank < 0)) grid_leave(ctl);
+  if (threadIdx.x == 0) grid_leave(ctl, gridDim.x);
 }
 
 // Clears a control block and records the XCD of this workgroup as its home.
