@@ -149,6 +149,12 @@ int ka_solver_set_tail(void* solver, int first, int32_t* level);
  * works alone (default 2000). *level receives the level in use, 0 for none.
  * No reference counterpart: identical iterates either way. */
 int ka_solver_set_grid(void* solver, int first, int limit_us, int32_t* level);
+/* How often a barrier between the workgroups of that cycle polls before it gives
+ * up (default 2^21, some 0.6 s; 0: at the first poll that does not find it
+ * passed). All of them are running by then, so none should; the solve that
+ * finds one given up is an error, and the cycle is off until ka_solver_set_grid
+ * or ka_solver_set_tail asks for it again. */
+int ka_solver_set_grid_polls(void* solver, int polls);
 /* The tail autotuner: times `repeats` V-cycles on the refreshed operator for
  * each admissible first level (and none) and keeps the fastest in *level.
  * The iterates are identical whichever is chosen. No reference counterpart. */

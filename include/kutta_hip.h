@@ -392,7 +392,8 @@ typedef enum kh_kernel {
      workgroups as `table` says (parts x count kh_grid_part); levels [grid,
      count), of at most KH_GRID_BOTTOM_ROWS rows each, belong to the first
      workgroup alone. limit_us: how long workgroups wait for each other before
-     one of them does the whole cycle alone (0: at once).
+     one of them does the whole cycle alone (0: at once). A barrier between
+     them that gives up leaves a wrong `out` and is counted in the report.
      levels,table,ctl,count,grid,pre,post,coarse_sweeps,parts,lds_words,
      limit_us,rhs,out,status (n = 1). */
   KH_GRID_INIT,                  /* ctl (n = 1) */
@@ -510,6 +511,15 @@ typedef struct kh_grid_part {
  * neighbouring lanes start on different LDS banks. */
 #define KH_GRID_CHUNKS(chunks) ((chunks) > 3 ? (chunks) | 1 : (chunks))
 #define KH_GRID_CTL_WORDS 160
+/* Words of a control block that INIT sets and its owner may change between
+ * launches: the polls a barrier makes before it gives up (2^21), and the device
+ * address (64 bits) of KH_GRID_REPORT_WORDS counters that CYCLE adds to (0: none):
+ * launches in which a barrier gave up. HOME is the XCD that INIT ran on. */
+#define KH_GRID_CTL_HOME 96
+#define KH_GRID_CTL_POLLS 97
+#define KH_GRID_CTL_REPORT 98
+#define KH_GRID_REPORT_GIVEN_UP 0
+#define KH_GRID_REPORT_WORDS 1
 #define KH_GRID_POOL_WORDS 39936
 
 /* Device::launch (device.hpp:205; cuda_device.cu:132-140): runs kernel `kernel`

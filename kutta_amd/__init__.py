@@ -123,6 +123,7 @@ def host_lib() -> C.CDLL:
         lib.ka_solver_host_waits.argtypes = [vp]
         lib.ka_solver_set_tail.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_grid.argtypes = [vp, i32, i32, pi32]
+        lib.ka_solver_set_grid_polls.argtypes = [vp, i32]
         lib.ka_solver_set_restart.argtypes = [vp, i32]
         lib.ka_solver_set_direct.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_dense_tolerance.argtypes = [vp, dbl]
@@ -912,6 +913,11 @@ class LinearSolver:
         level = C.c_int32(0)
         _check_host(host_lib().ka_solver_set_grid(self.handle, int(first), int(limit_us), C.byref(level)))
         return level.value
+
+    def set_grid_polls(self, polls: int = 1 << 21) -> None:
+        """How often a barrier of the multi-workgroup V-cycle polls before it
+        gives up; the solve that finds one given up raises."""
+        _check_host(host_lib().ka_solver_set_grid_polls(self.handle, int(polls)))
 
     def __del__(self):
         try:

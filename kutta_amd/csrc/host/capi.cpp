@@ -308,6 +308,9 @@ int ka_solver_set_tail(void* s, int first, int* level) {
     if (level) *level = used;
   });
 }
+int ka_solver_set_grid_polls(void* s, int polls) {
+  return guard([&] { static_cast<Solver*>(s)->solver.set_grid_polls(polls); });
+}
 int ka_solver_set_grid(void* s, int first, int limit_us, int32_t* level) {
   return guard([&] {
     const int used = static_cast<Solver*>(s)->solver.set_grid(first, limit_us);

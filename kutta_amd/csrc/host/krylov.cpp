@@ -124,12 +124,18 @@ struct KrylovSolver::Impl {
   DeviceArray<kh_grid_level> grid_levels;
   DeviceArray<kh_grid_part> grid_table;
   DeviceArray<std::uint32_t> grid_ctl;
+  int grid_polls = 1 << 21;  // what its barriers wait before they give up
+  Index grid_given_up = 0;   // launches that did, as last seen
 
   Impl(HipDevice& d, SolverKind k, const CsrHost& a, const AmgOptions& o)
       : dev(d), kind(k), options(o),
         amg(k == SolverKind::AmgPcg || k == SolverKind::AmgBicgstab || k == SolverKind::AmgFgmres),
         nullspace(o.nullspace == NullSpace::Constant), n(a.n_rows), nnz(a.nnz()) {
     validate_host(a);
+    // The solver's status, and what the multi-workgroup cycle counts: one
+    // poll reads both.
+    status = DeviceArray<Index>(dev, 3 + KH_GRID_REPORT_WORDS);
+    dev.fill_int(status.data(), 0, status.size());
     if (amg) {
       KA_REQUIRE(options.pre_sweeps > 0 && options.post_sweeps > 0 && options.coarse_sweeps > 0 &&
                      options.coarse_rows >= 1 && options.max_levels >= 1 &&
@@ -160,10 +166,8 @@ struct KrylovSolver::Impl {
       zs = DeviceArray<float>(dev, n);
     }
     scalars = DeviceArray<float>(dev, 24);
-    status = DeviceArray<Index>(dev, 3);
     projection = DeviceArray<float>(dev, 2);
     dev.fill(scalars.data(), 0.0f, 24);
-    dev.fill_int(status.data(), 0, 3);
   }
   bool bicg() const { return kind == SolverKind::BicgstabJacobi || kind == SolverKind::AmgBicgstab; }
   bool gmres() const { return kind == SolverKind::FgmresJacobi || kind == SolverKind::AmgFgmres; }
@@ -646,8 +650,26 @@ struct KrylovSolver::Impl {
     if (grid_ctl.empty()) {
       grid_ctl = DeviceArray<std::uint32_t>(dev, KH_GRID_CTL_WORDS);
       dev.launch(KH_GRID_INIT, 1, {grid_ctl});
+      const Index* report = status.data() + 3;
+      ok(kh_upload(dev.raw(), grid_ctl.data() + KH_GRID_CTL_REPORT, &report, sizeof report));
+      set_grid_polls(grid_polls);
     }
     grid_first = first;
+  }
+  void set_grid_polls(int polls) {
+    grid_polls = polls;
+    if (!grid_ctl.empty()) dev.fill_int(grid_ctl.data() + KH_GRID_CTL_POLLS, polls, 1);
+  }
+  // What the launches since the last look counted (`report` as downloaded with
+  // the status). After a barrier that gave up the iterate is wrong: the cycle
+  // is left off from here on and the caller told.
+  void look_at_grid(const Index* report) {
+    const Index given_up = report[KH_GRID_REPORT_GIVEN_UP];
+    if (given_up == grid_given_up) return;
+    grid_given_up = given_up;
+    grid_request = 0;
+    plan_tail();
+    throw Error("AMG: a barrier of the multi-workgroup cycle gave up; the cycle is off now");
   }
   void grid_cycle(const float* b, float* x, const int* st) {
     dev.launch(KH_GRID_CYCLE, 1,
@@ -1052,6 +1074,7 @@ struct KrylovSolver::Impl {
   std::array<Index, 3> poll() {
     ++waits;
     const auto host = status.download();
+    look_at_grid(host.data() + 3);
     return {host[0], host[1], host[2]};
   }
   void dot_into(const float* x, const float* y, int offset) {
@@ -1489,6 +1512,10 @@ int KrylovSolver::set_grid(int first, int limit_us) {
   I.plan_tail();
   return I.grid_first;
 }
+void KrylovSolver::set_grid_polls(int polls) {
+  KA_REQUIRE(polls >= 0, "AMG: the polls of the multi-workgroup cycle's barriers must not be negative");
+  impl_->set_grid_polls(polls);
+}
 
 // The coarse-tail autotuner (no reference counterpart): times `repeats`
 // V-cycles for each admissible first level of the tail, and for none, keeps
@@ -1661,6 +1688,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
       best_grid = int(i);
     }
   }
+  I.poll();
   I.grid_request = best_grid;
   I.tail_request = best;
   I.plan_tail();

@@ -103,6 +103,10 @@ class KrylovSolver {
   // limit_us is how long its workgroups wait for each other before one works
   // alone. Returns the level in use, 0 for none (iterates are the same).
   int set_grid(int first, int limit_us);
+  // How often a barrier between those workgroups polls before it gives up
+  // (default 2^21): the solve that finds one given up throws, and the cycle is
+  // off until set_grid or set_tail(-1) asks for it again.
+  void set_grid_polls(int polls);
   // Times `repeats` V-cycles per admissible tail level (and none) on the
   // refreshed operator and keeps the fastest; returns it. Identical iterates
   // either way. No reference counterpart.

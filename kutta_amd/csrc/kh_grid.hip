@@ -64,10 +64,13 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // kh_grid_gather.hpp uses it; the limit is in ticks of the 100 MHz clock.
 struct GridCtl {
   unsigned *arrived, *settled, *bar, *home, *left;
+  unsigned polls;
+  int* report;
   long limit;
   long long start = 0;
   __device__ GridCtl(unsigned* w, long limit_ticks)
-      : arrived(w), settled(w + 32), bar(w + 64), home(w + 96), left(w + 128), limit(limit_ticks) {}
+      : arrived(w), settled(w + 32), bar(w + 64), home(w + KH_GRID_CTL_HOME), left(w + 128),
+        polls(w[KH_GRID_CTL_POLLS]), report(*reinterpret_cast<int**>(w + KH_GRID_CTL_REPORT)), limit(limit_ticks) {}
   __device__ static unsigned add(unsigned* p, unsigned v) {
     return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -88,11 +91,16 @@ struct GridCtl {
     for (unsigned* p : {bar, left, settled, arrived})
       __hip_atomic_store(p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  __device__ void count(int what) const {
+    if (report != nullptr) __hip_atomic_fetch_add(report + what, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 };
 
 // Barrier over the members: all of them are running (grid_enter), and each
-// passes the same barriers, so the wait ends; it is bounded all the same.
-constexpr unsigned kBarrierSpins = 1u << 21;  // of some 0.3 us each
+// passes the same barriers, so the wait ends. It is bounded all the same: after
+// `polls` polls of some 0.3 us each a member gives up, which opens this and the
+// launch's later barriers to all and is reported, since the iterate is wrong.
+constexpr unsigned kGivenUp = 1u << 31, kBarrierPolls = 1u << 21;
 __device__ __forceinline__ void grid_sync(const GridCtl& c, int parts, unsigned& passed) {
   stores_done();
   __syncthreads();
@@ -100,8 +108,11 @@ __device__ __forceinline__ void grid_sync(const GridCtl& c, int parts, unsigned&
   if (threadIdx.x == 0) {
     GLOBAL unsigned* bar = (GLOBAL unsigned*)c.bar;
     __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (unsigned spin = 0; ctl_load(c.bar) < passed && spin < kBarrierSpins; ++spin) {
-    }
+    unsigned polls = 0, seen;
+    while ((seen = ctl_load(c.bar)) < passed && polls < c.polls) ++polls;
+    if (seen < passed &&
+        (__hip_atomic_fetch_or(bar, kGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kGivenUp) == 0)
+      c.count(KH_GRID_REPORT_GIVEN_UP);
   }
   __syncthreads();
 }
@@ -511,7 +522,10 @@ __global__ void __launch_bounds__(kGridThreads) k_grid_cycle(const CycleArgs A) 
 __global__ void k_grid_init(unsigned* ctl) {
   for (int i = threadIdx.x; i < KH_GRID_CTL_WORDS; i += blockDim.x) ctl[i] = 0;
   __syncthreads();
-  if (threadIdx.x == 0) ctl[96] = xcc_id();
+  if (threadIdx.x == 0) {
+    ctl[KH_GRID_CTL_HOME] = xcc_id();
+    ctl[KH_GRID_CTL_POLLS] = kBarrierPolls;
+  }
 }
 
 void allow_lds(kh_device* d) {

@@ -99,3 +99,34 @@ def test_grid_cycle_follows_new_values_and_limits(device):
         solver.solve(matrix, x, b, SolveControl(1e-6, 0.0, 300))
         out.append(x.download())
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+def test_a_barrier_that_gives_up_is_an_error(device):
+    """With no polls at all the first workgroup at a barrier gives up: every
+    launch still ends, the solve raises, and the cycle is off. Asked for again,
+    with its polls back, it gives the bits it gave before."""
+    p = oracle.pressure_problem(18, 17, 16).csr()
+    host = kutta_amd.CsrMatrixHost(p.row_ptr, p.col, p.diag, p.val)
+    matrix = kutta_amd.upload(device, host)
+    solver = kutta_amd.make_amg_solver(SolverKind.AmgPcg, device, host, AmgOptions(aggregation_passes=2, structure=M))
+    solver.refresh(matrix)
+    b = device.upload(np.random.default_rng(5).standard_normal(p.n_rows).astype(np.float32))
+
+    def run():
+        x = device.alloc(p.n_rows)
+        x.fill(np.float32(0))
+        solver.solve(matrix, x, b, SolveControl(1e-6, 0.0, 300))
+        return x.download().view(np.uint32)
+
+    want = run()
+    assert "multi-workgroup" in solver.plan()
+    for graphs in (True, False):
+        solver.set_graphs(graphs)
+        solver.set_grid_polls(0)
+        with pytest.raises(kutta_amd.KuttaError, match="gave up"):
+            run()
+        assert "multi-workgroup" not in solver.plan()
+        assert np.array_equal(run(), want)
+        solver.set_grid_polls()
+        assert solver.set_grid(-1) >= 1
+        assert np.array_equal(run(), want)
