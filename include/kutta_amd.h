@@ -155,6 +155,9 @@ int ka_solver_set_grid(void* solver, int first, int limit_us, int32_t* level);
  * finds one given up is an error, and the cycle is off until ka_solver_set_grid
  * or ka_solver_set_tail asks for it again. */
 int ka_solver_set_grid_polls(void* solver, int polls);
+/* out[3]: that cycle's launches so far, by its workgroups together, by one alone
+ * (the others did not meet it in time), and with a barrier given up. */
+int ka_solver_grid_report(void* solver, int32_t* out);
 /* The tail autotuner: times `repeats` V-cycles on the refreshed operator for
  * each admissible first level (and none) and keeps the fastest in *level.
  * The iterates are identical whichever is chosen. No reference counterpart. */

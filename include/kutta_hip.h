@@ -514,12 +514,16 @@ typedef struct kh_grid_part {
 /* Words of a control block that INIT sets and its owner may change between
  * launches: the polls a barrier makes before it gives up (2^21), and the device
  * address (64 bits) of KH_GRID_REPORT_WORDS counters that CYCLE adds to (0: none):
- * launches in which a barrier gave up. HOME is the XCD that INIT ran on. */
+ * launches in which a barrier gave up, that ran together, and in which one
+ * workgroup worked alone. HOME is the XCD whose workgroups work, at first the
+ * one that INIT ran on. */
 #define KH_GRID_CTL_HOME 96
 #define KH_GRID_CTL_POLLS 97
 #define KH_GRID_CTL_REPORT 98
 #define KH_GRID_REPORT_GIVEN_UP 0
-#define KH_GRID_REPORT_WORDS 1
+#define KH_GRID_REPORT_TOGETHER 1
+#define KH_GRID_REPORT_ALONE 2
+#define KH_GRID_REPORT_WORDS 3
 #define KH_GRID_POOL_WORDS 39936
 
 /* Device::launch (device.hpp:205; cuda_device.cu:132-140): runs kernel `kernel`

@@ -124,6 +124,7 @@ def host_lib() -> C.CDLL:
         lib.ka_solver_set_tail.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_grid.argtypes = [vp, i32, i32, pi32]
         lib.ka_solver_set_grid_polls.argtypes = [vp, i32]
+        lib.ka_solver_grid_report.argtypes = [vp, pi32]
         lib.ka_solver_set_restart.argtypes = [vp, i32]
         lib.ka_solver_set_direct.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_dense_tolerance.argtypes = [vp, dbl]
@@ -918,6 +919,13 @@ class LinearSolver:
         """How often a barrier of the multi-workgroup V-cycle polls before it
         gives up; the solve that finds one given up raises."""
         _check_host(host_lib().ka_solver_set_grid_polls(self.handle, int(polls)))
+
+    def grid_report(self) -> dict:
+        """The multi-workgroup V-cycle's launches so far: by its workgroups
+        together, by one alone, and with a barrier given up."""
+        out = (C.c_int32 * 3)()
+        _check_host(host_lib().ka_solver_grid_report(self.handle, out))
+        return {"together": out[0], "alone": out[1], "given_up": out[2]}
 
     def __del__(self):
         try:

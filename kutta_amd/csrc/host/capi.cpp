@@ -308,6 +308,12 @@ int ka_solver_set_tail(void* s, int first, int* level) {
     if (level) *level = used;
   });
 }
+int ka_solver_grid_report(void* s, int32_t* out) {
+  return guard([&] {
+    const auto report = static_cast<Solver*>(s)->solver.grid_report();
+    std::copy(report.begin(), report.end(), out);
+  });
+}
 int ka_solver_set_grid_polls(void* s, int polls) {
   return guard([&] { static_cast<Solver*>(s)->solver.set_grid_polls(polls); });
 }

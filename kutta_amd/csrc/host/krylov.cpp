@@ -1512,6 +1512,11 @@ int KrylovSolver::set_grid(int first, int limit_us) {
   I.plan_tail();
   return I.grid_first;
 }
+std::array<Index, 3> KrylovSolver::grid_report() const {
+  const auto host = impl_->status.download();
+  const Index* report = host.data() + 3;
+  return {report[KH_GRID_REPORT_TOGETHER], report[KH_GRID_REPORT_ALONE], report[KH_GRID_REPORT_GIVEN_UP]};
+}
 void KrylovSolver::set_grid_polls(int polls) {
   KA_REQUIRE(polls >= 0, "AMG: the polls of the multi-workgroup cycle's barriers must not be negative");
   impl_->set_grid_polls(polls);
@@ -1815,9 +1820,13 @@ std::string KrylovSolver::plan() const {
             : impl_->coarse_sweeps_mode == 2 && L.back().resident_cap > 0 ? "register-resident sweeps"
                                                                             : "one-workgroup sweeps");
   out << "; tail from level " << impl_->tail_first;
-  if (impl_->grid_first > 0)
-    out << ", multi-workgroup cycle from level " << impl_->grid_first << " (" << impl_->grid_plan.parts
-        << " workgroups)";
+  if (impl_->grid_first > 0) {
+    const GridPlan& g = impl_->grid_plan;
+    out << ", multi-workgroup cycle from level " << impl_->grid_first << " (" << g.parts << " workgroups, " << g.grid
+        << " of " << g.count << " levels shared, row sums";
+    for (int k = 0; k < g.count; ++k) out << (k ? "," : " ") << (g.table[std::size_t(k)].mode ? "split" : "whole");
+    out << ")";
+  }
   out << "; longest row per level";
   for (std::size_t i = 0; i < L.size(); ++i) out << (i ? "," : " ") << L[i].max_row;
   out << "; sweeps per level";

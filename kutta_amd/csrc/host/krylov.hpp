@@ -5,6 +5,7 @@
 // the host only reads a 3-int status once per batch.
 #pragma once
 
+#include <array>
 #include <memory>
 #include <string>
 #include <vector>
@@ -107,6 +108,9 @@ class KrylovSolver {
   // (default 2^21): the solve that finds one given up throws, and the cycle is
   // off until set_grid or set_tail(-1) asks for it again.
   void set_grid_polls(int polls);
+  // Launches of that cycle so far: by its workgroups together, by one alone,
+  // and with a barrier given up.
+  std::array<Index, 3> grid_report() const;
   // Times `repeats` V-cycles per admissible tail level (and none) on the
   // refreshed operator and keeps the fastest; returns it. Identical iterates
   // either way. No reference counterpart.

@@ -512,6 +512,9 @@ __global__ void __launch_bounds__(kGridThreads) k_grid_cycle(const CycleArgs A) 
   if (threadIdx.x == 0) place = grid_enter(ctl, gridDim.x, A.parts, xcc_id() == ctl_load(ctl.home));
   __syncthreads();
   const GridRole role = GridRole(__builtin_amdgcn_readfirstlane(int(place.role)));
+  // Counted at once, so that the cycle hides it.
+  if (threadIdx.x == 0 && role == GridRole::Solo) ctl.count(KH_GRID_REPORT_ALONE);
+  if (threadIdx.x == 0 && role == GridRole::Member && place.rank == 0) ctl.count(KH_GRID_REPORT_TOGETHER);
   if (role == GridRole::Member) member_cycle(A, ctl, __builtin_amdgcn_readfirstlane(place.rank));
   else if (role == GridRole::Solo) solo_cycle(A);
   __syncthreads();

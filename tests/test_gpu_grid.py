@@ -3,7 +3,12 @@ it replaces: bitwise-identical iterates, iteration counts and residuals from
 every admissible first level, through graph replays and direct launches, with
 its workgroups together and with one working alone (a wait of zero), on
 hierarchies that end in the few-row coarse solve, in coarse sweeps, and in
-levels too large for the one-workgroup part."""
+levels too large for the one-workgroup part. Both ways give the same bits, so
+which of them ran is read from the cycle's own counts, and which forms a plan
+has from plan(): each case states those it is there for."""
+import ctypes as C
+import re
+
 import numpy as np
 import pytest
 
@@ -14,27 +19,31 @@ from kutta_amd import AmgCycle, AmgOptions, OperatorStructure, SolveControl, Sol
 pytestmark = pytest.mark.gpu
 M = OperatorStructure.SymmetricMMatrix
 
+# Last, the forms of a case's plans: workgroups, "bottom" (levels the first workgroup
+# does alone) or "shared" (no such level), and how rows are summed ("split":
+# products first; "whole": entry by entry, above 512 rows a workgroup).
 CASES = [
-    ("poisson V(5,5)", lambda: oracle.poisson(30, 28, 26), SolverKind.AmgPcg, AmgOptions()),
+    ("poisson V(5,5)", lambda: oracle.poisson(30, 28, 26), SolverKind.AmgPcg, AmgOptions(), "16 bottom split"),
     ("ragged rows V(2,2)", lambda: oracle.poisson(33, 31, 29, 1.0, random=True), SolverKind.AmgPcg,
-     AmgOptions(pre_sweeps=2, post_sweeps=2, aggregation_passes=2)),
-    ("V(1,1)", lambda: oracle.poisson(23, 21, 19), SolverKind.AmgPcg, AmgOptions(pre_sweeps=1, post_sweeps=1)),
+     AmgOptions(pre_sweeps=2, post_sweeps=2, aggregation_passes=2), "16 shared split"),
+    ("V(1,1)", lambda: oracle.poisson(23, 21, 19), SolverKind.AmgPcg, AmgOptions(pre_sweeps=1, post_sweeps=1),
+     "16 bottom split"),
     ("pressure, coarse sweeps", lambda: oracle.pressure_problem(18, 17, 16).csr(), SolverKind.AmgPcg,
-     AmgOptions(aggregation_passes=2, coarse_rows=400, structure=M)),
+     AmgOptions(aggregation_passes=2, coarse_rows=400, structure=M), "16 bottom split"),
     ("pressure, stalled coarse levels", lambda: oracle.pressure_problem(24, 23, 22).csr(), SolverKind.AmgPcg,
-     AmgOptions(aggregation_passes=2, structure=M)),
+     AmgOptions(aggregation_passes=2, structure=M), "16 32 bottom split whole"),
     ("anisotropic, pair aggregates", lambda: oracle.poisson(32, 32, 32, 100), SolverKind.AmgPcg,
-     AmgOptions(aggregation_passes=1, max_levels=4)),
+     AmgOptions(aggregation_passes=1, max_levels=4), "16 shared split whole"),
     ("bicgstab V(2,3)", lambda: oracle.poisson(52, 47, 1, 1.0, wind=2.0), SolverKind.AmgBicgstab,
-     AmgOptions(pre_sweeps=2, post_sweeps=3, aggregation_passes=2)),
+     AmgOptions(pre_sweeps=2, post_sweeps=3, aggregation_passes=2), "16 bottom split"),
     ("K-cycle", lambda: oracle.pressure_problem(20, 19, 18).csr(), SolverKind.AmgPcg,
      AmgOptions(pre_sweeps=1, post_sweeps=1, coarse_sweeps=4, aggregation_passes=2, structure=M, cycle=AmgCycle.K,
-                k_min_rows=5000)),
+                k_min_rows=5000), "16 bottom split"),
 ]
 
 
-@pytest.mark.parametrize("name,make,kind,opts", CASES, ids=[c[0] for c in CASES])
-def test_grid_cycle_matches_level_launches(device, name, make, kind, opts):
+@pytest.mark.parametrize("name,make,kind,opts,forms", CASES, ids=[c[0] for c in CASES])
+def test_grid_cycle_matches_level_launches(device, name, make, kind, opts, forms):
     a = make()
     host = kutta_amd.CsrMatrixHost(a.row_ptr, a.col, a.diag, a.val)
     matrix = kutta_amd.upload(device, host)
@@ -53,7 +62,7 @@ def test_grid_cycle_matches_level_launches(device, name, make, kind, opts):
     solver.set_tail(0)
     st0, x0 = run()
     assert "multi-workgroup" not in solver.plan()
-    tried = 0
+    seen = set()
     for first in range(1, len(solver.levels())):
         try:
             assert solver.set_grid(first) == first
@@ -64,12 +73,20 @@ def test_grid_cycle_matches_level_launches(device, name, make, kind, opts):
             solver.set_graphs(graphs)
             solver.set_grid(first, limit)
             assert f"multi-workgroup cycle from level {first}" in solver.plan()
+            before = solver.grid_report()
             for _ in range(2):
                 st, x = run()
                 assert (st.iterations, st.final_residual) == (st0.iterations, st0.final_residual)
                 assert np.array_equal(x.view(np.uint32), x0.view(np.uint32))
-        tried += 1
-    assert tried >= 1
+            ran = {k: v - before[k] for k, v in solver.grid_report().items()}
+            assert ran["given_up"] == 0
+            if limit > 0:
+                assert ran["together"] >= st0.iterations and ran["alone"] == 0
+            else:
+                assert ran["alone"] > 0
+        plan = re.search(r"\((\d+) workgroups, (\d+) of (\d+) levels shared, row sums ([a-z,]+)\)", solver.plan())
+        seen |= {plan.group(1), "shared" if plan.group(2) == plan.group(3) else "bottom", *plan.group(4).split(",")}
+    assert seen == set(forms.split())
 
 
 def test_grid_cycle_follows_new_values_and_limits(device):
@@ -130,3 +147,85 @@ def test_a_barrier_that_gives_up_is_an_error(device):
         solver.set_grid_polls()
         assert solver.set_grid(-1) >= 1
         assert np.array_equal(run(), want)
+
+
+class Level(C.Structure):
+    _fields_ = [(k, C.c_void_p) for k in ("row_ptr", "col", "val", "inverse", "member_offsets", "members", "aggregate",
+                                          "place", "slot", "local_col", "x", "w", "b")] + [
+                (k, C.c_int32) for k in ("rows", "pad")]
+
+
+class Part(C.Structure):
+    _fields_ = [(k, C.c_int32) for k in ("first", "rows", "window", "window_rows", "slot0", "slots", "mode", "lds",
+                                         "terms", "iterates")]
+
+
+def one_level_plan(row_ptr, col, parts):
+    """KH_GRID_CYCLE's tables for one shared level, as kutta_hip.h states them."""
+    n = len(row_ptr) - 1
+    place, slot, local, table = np.zeros(n, np.uint16), [], [], []
+    for p in range(parts):
+        first, last = n * p // parts, n * (p + 1) // parts
+        cols = col[row_ptr[first]:row_ptr[last]]
+        low, high = min(first, cols.min()), max(last, cols.max() + 1)
+        slot0 = len(slot)
+        for i in range(first, last):
+            entries = list(range(row_ptr[i], row_ptr[i + 1]))
+            chunks = (len(entries) + 3) // 4
+            pad = 4 * (chunks | 1 if chunks > 3 else chunks) - len(entries)
+            place[i] = len(slot) - slot0
+            slot += entries + [-1] * pad
+            local += [col[j] - low for j in entries] + [0xffff] * pad
+        table.append(Part(first, last - first, low, high - low, slot0, len(slot) - slot0, 1))
+    window = (max(t.window_rows for t in table) + 3) // 4 * 4
+    base = window + 2 * max(t.slots for t in table)
+    for t in table:
+        t.terms, t.lds = window, base
+    words = base + max(t.slots + t.slots // 2 + 3 * t.rows for t in table)
+    assert words <= 39936 and all(t.slots % 4 == 0 and t.window_rows < 0xffff for t in table)
+    return place, np.array(slot, np.int32), np.array(local, np.uint16), table, (words + 3) // 4 * 4
+
+
+@pytest.mark.parametrize("parts", [1, 2, 5, 16, 32])
+def test_launch_with_and_without_workgroups_on_the_home_xcd(device, parts):
+    """The launch by itself on one level, five sweeps: its workgroups together,
+    and, with a home that no XCD has, one of them alone from the first launch
+    on, without a wait and without counters. Both as the sweeps' own launches."""
+    a = oracle.poisson(11, 10, 9, 1.0, random=True)
+    n, K = a.n_rows, kutta_amd.Kernel
+    row_ptr, col = np.asarray(a.row_ptr, np.int32), np.asarray(a.col, np.int32)
+    rng = np.random.default_rng(parts)
+    rows, cols = device.upload(row_ptr), device.upload(col)
+    vals, b = device.upload(np.asarray(a.val, np.float32)), device.upload(rng.standard_normal(n).astype(np.float32))
+    inverse, status = device.upload((0.1 + 0.1 * rng.random(n)).astype(np.float32)), device.upload(np.zeros(3, np.int32))
+    x, w = device.alloc(n), device.alloc(n)
+    device.launch(K.fused_smooth_from_zero, n, rows, cols, vals, b, inverse, x, status)
+    for _ in range(2):
+        device.launch(K.amg_smooth, n, rows, cols, vals, x, b, inverse, w, status)
+        device.launch(K.amg_smooth, n, rows, cols, vals, w, b, inverse, x, status)
+    want = x.download().view(np.uint32)
+
+    place, slot, local, table, words = one_level_plan(row_ptr, col, parts)
+    arrays = [device.upload(v) for v in (place, slot, local)]
+    level = Level(rows.ptr, cols.ptr, vals.ptr, inverse.ptr, 0, 0, 0, *(v.ptr for v in arrays), x.ptr, w.ptr, b.ptr, n, 0)
+    levels = device.upload(np.frombuffer(bytes(level), np.uint8))
+    parts_table = device.upload(np.frombuffer(b"".join(bytes(t) for t in table), np.uint8))
+    ctl, report = device.alloc(160, np.uint32), device.upload(np.zeros(3, np.int32))
+    device.launch(K.grid_init, 1, ctl)
+    block = ctl.download()
+    home = int(block[96])
+    assert not block[:96].any() and not block[98:].any()
+    given_up, together, alone = 0, 0, 0
+    for on, counted in ((home, True), (15, True), (home, True), (15, False), (home, False)):
+        print(f"[grid] {parts} parts, home {on}", flush=True)
+        block[96] = on
+        block[98:100] = np.array([report.ptr if counted else 0], np.uint64).view(np.uint32)
+        ctl.upload(block)
+        for _ in range(3):
+            out = device.upload(np.full(n, np.nan, np.float32))
+            device.launch(K.grid_cycle, 1, levels, parts_table, ctl, 1, 1, 1, 1, 5, parts, words, 2000, b, out, status)
+            assert np.array_equal(out.download().view(np.uint32), want)
+            assert np.array_equal(ctl.download(), block)  # clear for the next launch
+        together += 3 * (counted and on == home)
+        alone += 3 * (counted and on != home)
+        assert list(report.download()) == [given_up, together, alone]
