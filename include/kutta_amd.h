@@ -147,7 +147,10 @@ int ka_solver_set_tail(void* solver, int first, int32_t* level);
  * error if levels k.. do not fit; needs the tail automatic, which it sets).
  * limit_us: how long its workgroups wait for each other before one of them
  * works alone (default 2000). *level receives the level in use, 0 for none.
- * No reference counterpart: identical iterates either way. */
+ * Unless requested by level, it is not used on a device whose launches do not go
+ * round-robin over 8 XCDs, and a solve in which one workgroup worked alone three
+ * times (another stream's kernels hold the card) goes on without it, as do the
+ * next 256. No reference counterpart: identical iterates either way. */
 int ka_solver_set_grid(void* solver, int first, int limit_us, int32_t* level);
 /* How often a barrier between the workgroups of that cycle polls before it gives
  * up (default 2^21, some 0.6 s; 0: at the first poll that does not find it

@@ -516,10 +516,13 @@ typedef struct kh_grid_part {
  * address (64 bits) of KH_GRID_REPORT_WORDS counters that CYCLE adds to (0: none):
  * launches in which a barrier gave up, that ran together, and in which one
  * workgroup worked alone. HOME is the XCD whose workgroups work, at first the
- * one that INIT ran on. */
+ * one that INIT ran on, and SPREAD how many workgroups of a launch of
+ * 8 KH_GRID_MAX_PARTS found themselves there: where it is KH_GRID_MAX_PARTS,
+ * launches go round-robin over 8 XCDs, as CYCLE's workgroups need to meet. */
 #define KH_GRID_CTL_HOME 96
 #define KH_GRID_CTL_POLLS 97
 #define KH_GRID_CTL_REPORT 98
+#define KH_GRID_CTL_SPREAD 100
 #define KH_GRID_REPORT_GIVEN_UP 0
 #define KH_GRID_REPORT_TOGETHER 1
 #define KH_GRID_REPORT_ALONE 2

@@ -126,6 +126,17 @@ struct KrylovSolver::Impl {
   DeviceArray<std::uint32_t> grid_ctl;
   int grid_polls = 1 << 21;  // what its barriers wait before they give up
   Index grid_given_up = 0;   // launches that did, as last seen
+  // Launches in which one workgroup worked alone cost the wait and then some
+  // milliseconds on one CU. Another stream's kernels on the card cause them, so
+  // after kGridMisses in one solve a cycle that nobody asked for by level rests
+  // for kGridRest solves, the tail or the levels' launches in its place.
+  static constexpr int kGridMisses = 3, kGridRest = 256;
+  bool grid_asked = false;
+  Index grid_alone = 0;  // as last seen
+  int grid_missed = 0;   // of this solve
+  int grid_rest = 0;     // solves left without the cycle, this one among them
+  bool grid_spread = false;  // launches go over the XCDs as the cycle needs
+  bool grid_on() const { return grid_first > 0 && !coarse_bf16 && grid_rest == 0; }
 
   Impl(HipDevice& d, SolverKind k, const CsrHost& a, const AmgOptions& o)
       : dev(d), kind(k), options(o),
@@ -604,6 +615,17 @@ struct KrylovSolver::Impl {
     grid_arrays.clear();
     grid_levels = DeviceArray<kh_grid_level>();
     grid_table = DeviceArray<kh_grid_part>();
+    grid_missed = grid_rest = 0;
+  }
+  // The control block, made on first use.
+  void grid_block() {
+    if (!grid_ctl.empty()) return;
+    grid_ctl = DeviceArray<std::uint32_t>(dev, KH_GRID_CTL_WORDS);
+    dev.launch(KH_GRID_INIT, 1, {grid_ctl});
+    const Index* report = status.data() + 3;
+    ok(kh_upload(dev.raw(), grid_ctl.data() + KH_GRID_CTL_REPORT, &report, sizeof report));
+    set_grid_polls(grid_polls);
+    grid_spread = grid_ctl.download()[KH_GRID_CTL_SPREAD] == KH_GRID_MAX_PARTS;
   }
   void pick_grid() {
     if (grid_request == 0) return;
@@ -613,7 +635,8 @@ struct KrylovSolver::Impl {
     }
     for (std::size_t i = 1; i + 1 < levels.size(); ++i)
       if (plan_grid_at(i, grid_plan, true)) {
-        use_grid(int(i));
+        grid_block();
+        if (grid_spread) use_grid(int(i));
         return;
       }
   }
@@ -647,13 +670,7 @@ struct KrylovSolver::Impl {
     }
     grid_levels = to_device(dev, table);
     grid_table = to_device(dev, grid_plan.table);
-    if (grid_ctl.empty()) {
-      grid_ctl = DeviceArray<std::uint32_t>(dev, KH_GRID_CTL_WORDS);
-      dev.launch(KH_GRID_INIT, 1, {grid_ctl});
-      const Index* report = status.data() + 3;
-      ok(kh_upload(dev.raw(), grid_ctl.data() + KH_GRID_CTL_REPORT, &report, sizeof report));
-      set_grid_polls(grid_polls);
-    }
+    grid_block();
     grid_first = first;
   }
   void set_grid_polls(int polls) {
@@ -664,7 +681,13 @@ struct KrylovSolver::Impl {
   // the status). After a barrier that gave up the iterate is wrong: the cycle
   // is left off from here on and the caller told.
   void look_at_grid(const Index* report) {
-    const Index given_up = report[KH_GRID_REPORT_GIVEN_UP];
+    const Index given_up = report[KH_GRID_REPORT_GIVEN_UP], alone = report[KH_GRID_REPORT_ALONE];
+    grid_missed += alone - grid_alone;
+    grid_alone = alone;
+    if (grid_missed >= kGridMisses && !grid_asked && grid_on()) {
+      drop_graphs();
+      grid_rest = kGridRest + 1;
+    }
     if (given_up == grid_given_up) return;
     grid_given_up = given_up;
     grid_request = 0;
@@ -829,7 +852,7 @@ struct KrylovSolver::Impl {
     Level& l = levels[index];
     float* w = l.r.data();
     CycleResult result;
-    const bool grid = grid_first > 0 && !coarse_bf16;
+    const bool grid = grid_on();
     if (fused && grid && int(index) == grid_first) {
       grid_cycle(b, x, st);
       return result;
@@ -1346,6 +1369,8 @@ struct KrylovSolver::Impl {
     SolveStats st;
     double target = 0;
     if (!solve_begin(a, x, b, c, st, target)) return st;
+    grid_missed = 0;
+    if (grid_rest > 0 && --grid_rest == 0) drop_graphs();
     if (kind == SolverKind::PcgJacobi || kind == SolverKind::AmgPcg) pcg(a, x, b, c, target, st);
     else if (bicg()) bicgstab(a, x, b, c, target, st);
     else if (gmres()) fgmres(a, x, b, c, target, st);
@@ -1487,7 +1512,10 @@ std::vector<SolveStats> KrylovSolver::solve_batched(const std::vector<KrylovSolv
 int KrylovSolver::set_tail(int first) {
   const int previous = impl_->tail_request;
   impl_->tail_request = first;
-  if (first < 0) impl_->grid_request = -1;
+  if (first < 0) {
+    impl_->grid_request = -1;
+    impl_->grid_asked = false;
+  }
   try {
     impl_->plan_tail();
   } catch (...) {
@@ -1507,6 +1535,7 @@ int KrylovSolver::set_grid(int first, int limit_us) {
                "AMG: levels from " + std::to_string(first) + " do not fit the multi-workgroup cycle");
   }
   I.grid_request = first;
+  I.grid_asked = first > 0;
   I.grid_limit_us = limit_us;
   if (first != 0) I.tail_request = -1;
   I.plan_tail();
@@ -1684,7 +1713,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
     I.tail_request = -1;
     I.grid_request = int(i);
     I.plan_tail();
-    if (I.grid_first == 0) continue;
+    if (I.grid_first == 0 || !I.grid_spread) continue;
     I.reset(0);
     const double secs = seconds([&] { I.apply(a, v.data(), out.data(), Tail::None); });
     if (secs < kKeep * best_s) {
@@ -1694,6 +1723,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
     }
   }
   I.poll();
+  I.grid_asked = false;
   I.grid_request = best_grid;
   I.tail_request = best;
   I.plan_tail();
@@ -1826,6 +1856,7 @@ std::string KrylovSolver::plan() const {
         << " of " << g.count << " levels shared, row sums";
     for (int k = 0; k < g.count; ++k) out << (k ? "," : " ") << (g.table[std::size_t(k)].mode ? "split" : "whole");
     out << ")";
+    if (impl_->grid_rest > 0) out << " resting for " << impl_->grid_rest - 1 << " more solves";
   }
   out << "; longest row per level";
   for (std::size_t i = 0; i < L.size(); ++i) out << (i ? "," : " ") << L[i].max_row;

@@ -102,7 +102,10 @@ class KrylovSolver {
   // The multi-workgroup V-cycle (KH_GRID_CYCLE): first < 0 picks its first
   // level automatically (the default), 0 turns it off, k requests level k;
   // limit_us is how long its workgroups wait for each other before one works
-  // alone. Returns the level in use, 0 for none (iterates are the same).
+  // alone. Picked automatically, it is not used where launches do not go over
+  // the XCDs as it needs, and after a solve in which one worked alone three
+  // times it rests for 256 solves. Returns the level in use, 0 for none
+  // (iterates are the same).
   int set_grid(int first, int limit_us);
   // How often a barrier between those workgroups polls before it gives up
   // (default 2^21): the solve that finds one given up throws, and the cycle is

@@ -530,6 +530,10 @@ __global__ void k_grid_init(unsigned* ctl) {
     ctl[KH_GRID_CTL_POLLS] = kBarrierPolls;
   }
 }
+// Counts the workgroups of a launch that are on the home XCD.
+__global__ void k_grid_spread(unsigned* ctl) {
+  if (threadIdx.x == 0 && xcc_id() == ctl[KH_GRID_CTL_HOME]) GridCtl::add(ctl + KH_GRID_CTL_SPREAD, 1);
+}
 
 void allow_lds(kh_device* d) {
   if (d->grid_ready) return;
@@ -541,6 +545,7 @@ void allow_lds(kh_device* d) {
 void l_grid_init(kh_device* d, int, const kh_arg* a) {
   allow_lds(d);  // not first under a capture
   k_grid_init<<<dim3(1), dim3(64), 0, d->stream>>>(static_cast<unsigned*>(buf(a, 0)));
+  k_grid_spread<<<dim3(8 * KH_GRID_MAX_PARTS), dim3(64), 0, d->stream>>>(static_cast<unsigned*>(buf(a, 0)));
 }
 // levels, table, ctl, count, grid, pre, post, coarse_sweeps, parts, lds_words,
 // limit_us, rhs, out, status

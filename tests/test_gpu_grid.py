@@ -149,6 +149,48 @@ def test_a_barrier_that_gives_up_is_an_error(device):
         assert np.array_equal(run(), want)
 
 
+def test_a_cycle_that_does_not_meet_rests(device):
+    """Picked automatically and given no time to meet, the cycle is worked
+    alone until the solve's next poll and then left off, for that solve and the
+    next 256; then it is tried again. Asked for by level it stays. Always the
+    same bits."""
+    a = oracle.poisson(17, 16, 15)
+    host = kutta_amd.CsrMatrixHost(a.row_ptr, a.col, a.diag, a.val)
+    matrix = kutta_amd.upload(device, host)
+    solver = kutta_amd.make_amg_solver(SolverKind.AmgPcg, device, host, AmgOptions(pre_sweeps=1, post_sweeps=1))
+    solver.refresh(matrix)
+    b = device.upload(np.random.default_rng(8).standard_normal(a.n_rows).astype(np.float32))
+
+    def run():
+        x = device.alloc(a.n_rows)
+        x.fill(np.float32(0))
+        assert solver.solve(matrix, x, b, SolveControl(1e-6, 0.0, 300)).iterations > 8  # more than one poll
+        return x.download().view(np.uint32), solver.grid_report()
+
+    first = solver.set_grid(-1)
+    want, report = run()
+    assert first >= 1 and report["together"] > 8 and report["alone"] == 0
+    solver.set_grid(-1, 0)
+    for k in range(3):
+        got, before = run()
+        assert np.array_equal(got, want)
+        assert f"resting for {256 - k} more solves" in solver.plan()
+        assert before["alone"] >= 3 and before["together"] == report["together"]
+    for _ in range(254):
+        got, after = run()
+        assert after == before
+    assert "resting for 0 more solves" in solver.plan() and np.array_equal(got, want)
+    got, after = run()
+    assert after["alone"] > before["alone"] and np.array_equal(got, want)
+    assert "resting for 256 more solves" in solver.plan()
+    solver.set_grid(first, 0)
+    for _ in range(2):
+        before = after
+        got, after = run()
+        assert after["alone"] > before["alone"] + 8 and np.array_equal(got, want)
+    assert "resting" not in solver.plan()
+
+
 class Level(C.Structure):
     _fields_ = [(k, C.c_void_p) for k in ("row_ptr", "col", "val", "inverse", "member_offsets", "members", "aggregate",
                                           "place", "slot", "local_col", "x", "w", "b")] + [
@@ -214,7 +256,8 @@ def test_launch_with_and_without_workgroups_on_the_home_xcd(device, parts):
     device.launch(K.grid_init, 1, ctl)
     block = ctl.download()
     home = int(block[96])
-    assert not block[:96].any() and not block[98:].any()
+    assert not block[:96].any() and not block[98:100].any() and not block[101:].any()
+    assert block[100] == 32  # of 256 workgroups: round-robin over 8 XCDs
     given_up, together, alone = 0, 0, 0
     for on, counted in ((home, True), (15, True), (home, True), (15, False), (home, False)):
         print(f"[grid] {parts} parts, home {on}", flush=True)
