@@ -881,7 +881,7 @@ def main() -> int:
     b = dev.upload(b_host)
     x = dev.alloc(problem.n_cells)
     control = SolveControl(rel_tol=1e-6, abs_tol=0.0, max_iter=2000)
-    print(f"[bench] {problem.n_cells} cells, nnz {problem.nnz}, {solver.describe()}, tail level {tail_level}", file=sys.stderr,
+    print(f"[bench] {problem.n_cells} cells, nnz {problem.nnz}, {solver.describe()}, tail level {tail_level}, grid level {solver.grid_level}", file=sys.stderr,
           flush=True)
 
     for _ in range(args.warmup):
@@ -1072,7 +1072,8 @@ def main() -> int:
             "hierarchy": solver.describe(),
             "plan": solver.plan(),
             "levels": solver.levels(),
-            "coarse_tail_level": tail_level,
+            "coarse_tail_level": 0 if solver.grid_level else tail_level,
+            "grid_cycle_level": solver.grid_level,
             "tail_autotune_s": round(autotune_s, 3),
             "iterations": st.iterations,
             "relative_residual": st.final_residual / st.initial_residual,

@@ -109,7 +109,8 @@ int ka_solver_solve_batched(void* const* solvers, void* const* matrices, float* 
                             int count, double rel_tol, double abs_tol, int max_iter, int interval, double* stats);
 int ka_solver_describe(void* solver, char* out, int capacity);
 /* The V-cycle forms the autotuner (ka_solver_autotune_tail) picked: the
- * restriction form per level, the coarsest level's sweeps, the tail level.
+ * restriction form per level, the coarsest level's sweeps, the tail's or the
+ * multi-workgroup cycle's level.
  * No reference counterpart; all forms give the same iterates. */
 int ka_solver_plan(void* solver, char* out, int capacity);
 /* Forces the plan: every level's restriction form (0 one kernel, 1 the same
@@ -138,13 +139,16 @@ int ka_solver_host_waits(void* solver);
 /* First AMG level of the one-workgroup coarse-grid tail (KH_FUSED_COARSE_TAIL)
  * on the fused path: first < 0 picks it automatically (the default), 0 turns
  * the tail off, k >= 1 requests level k (an error if levels k.. do not fit).
- * *level receives the level in use, 0 for none. No reference counterpart: the
- * iterates are those of the per-level launches either way. */
+ * *level receives the tail's first level, 0 for none; the automatic tail gives
+ * way to the multi-workgroup cycle below wherever that is in use
+ * (ka_solver_grid_level). No reference counterpart: the iterates are those of
+ * the per-level launches either way. */
 int ka_solver_set_tail(void* solver, int first, int32_t* level);
 /* First AMG level of the multi-workgroup V-cycle (KH_GRID_CYCLE), which takes
  * the automatic tail's place where its plan fits: first < 0 picks it
- * automatically (the default), 0 turns it off, k >= 1 requests level k (an
- * error if levels k.. do not fit; needs the tail automatic, which it sets).
+ * automatically (the default), 0 turns it off (until a call with another
+ * `first`), k >= 1 requests level k (an error if levels k.. do not fit; needs
+ * the tail automatic, which it sets).
  * limit_us: how long its workgroups wait for each other before one of them
  * works alone (default 2000). *level receives the level in use, 0 for none.
  * Unless requested by level, it is not used on a device whose launches do not go
@@ -152,6 +156,8 @@ int ka_solver_set_tail(void* solver, int first, int32_t* level);
  * times (another stream's kernels hold the card) goes on without it, as do the
  * next 256. No reference counterpart: identical iterates either way. */
 int ka_solver_set_grid(void* solver, int first, int limit_us, int32_t* level);
+/* That level as it is now, picked, requested or found by the autotuner. */
+int ka_solver_grid_level(void* solver);
 /* How often a barrier between the workgroups of that cycle polls before it gives
  * up (default 2^21, some 0.6 s; 0: at the first poll that does not find it
  * passed). All of them are running by then, so none should; the solve that
@@ -162,8 +168,12 @@ int ka_solver_set_grid_polls(void* solver, int polls);
  * (the others did not meet it in time), and with a barrier given up. */
 int ka_solver_grid_report(void* solver, int32_t* out);
 /* The tail autotuner: times `repeats` V-cycles on the refreshed operator for
- * each admissible first level (and none) and keeps the fastest in *level.
- * The iterates are identical whichever is chosen. No reference counterpart. */
+ * each admissible first level (and none), and for the multi-workgroup cycle
+ * unless ka_solver_set_grid turned it off, and keeps the fastest. *level
+ * receives the tail's level, 0 for none, or -1 for that cycle: given to
+ * ka_solver_set_tail each chooses the same again (-1 the automatic one;
+ * ka_solver_set_grid with ka_solver_grid_level the very one). The iterates are
+ * identical whichever is chosen. No reference counterpart. */
 int ka_solver_autotune_tail(void* solver, void* matrix, int repeats, int32_t* level);
 /* Restart length m (1..63) of the FGMRES kinds. No reference counterpart. */
 int ka_solver_set_restart(void* solver, int m);

@@ -125,6 +125,7 @@ def host_lib() -> C.CDLL:
         lib.ka_solver_set_grid.argtypes = [vp, i32, i32, pi32]
         lib.ka_solver_set_grid_polls.argtypes = [vp, i32]
         lib.ka_solver_grid_report.argtypes = [vp, pi32]
+        lib.ka_solver_grid_level.argtypes = [vp]
         lib.ka_solver_set_restart.argtypes = [vp, i32]
         lib.ka_solver_set_direct.argtypes = [vp, i32, pi32]
         lib.ka_solver_set_dense_tolerance.argtypes = [vp, dbl]
@@ -828,9 +829,10 @@ class LinearSolver:
         _check_host(host_lib().ka_solver_learned_parameters(self.handle, t.ctypes.data, t.size, 1))
 
     def autotune_tail(self, a, repeats: int = 5) -> int:
-        """Time V-cycles for each admissible coarse-tail level (and none) on
-        the refreshed operator; keep and return the fastest (identical
-        iterates whichever)."""
+        """Time V-cycles for each admissible coarse-tail level (and none), and
+        for the multi-workgroup cycle unless it is off, on the refreshed
+        operator; keep the fastest and return the tail's level, 0 for none, or
+        -1 for that cycle (see grid_level). Identical iterates whichever."""
         level = C.c_int32()
         _check_host(host_lib().ka_solver_autotune_tail(self.handle, a.handle, int(repeats), C.byref(level)))
         return level.value
@@ -902,7 +904,8 @@ class LinearSolver:
 
     def set_tail(self, first: int = -1) -> int:
         """First level of the one-workgroup coarse-grid tail: -1 automatic,
-        0 off, k >= 1 level k. Returns the level in use (0: none)."""
+        0 off, k >= 1 level k. Returns the tail's level (0: none); the
+        automatic tail gives way to the multi-workgroup cycle (grid_level)."""
         level = C.c_int32(0)
         _check_host(host_lib().ka_solver_set_tail(self.handle, int(first), C.byref(level)))
         return level.value
@@ -914,6 +917,11 @@ class LinearSolver:
         level = C.c_int32(0)
         _check_host(host_lib().ka_solver_set_grid(self.handle, int(first), int(limit_us), C.byref(level)))
         return level.value
+
+    @property
+    def grid_level(self) -> int:
+        """The multi-workgroup V-cycle's first level now (0: none)."""
+        return host_lib().ka_solver_grid_level(self.handle)
 
     def set_grid_polls(self, polls: int = 1 << 21) -> None:
         """How often a barrier of the multi-workgroup V-cycle polls before it

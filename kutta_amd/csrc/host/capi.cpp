@@ -308,6 +308,7 @@ int ka_solver_set_tail(void* s, int first, int* level) {
     if (level) *level = used;
   });
 }
+int ka_solver_grid_level(void* s) { return static_cast<Solver*>(s)->solver.grid_level(); }
 int ka_solver_grid_report(void* s, int32_t* out) {
   return guard([&] {
     const auto report = static_cast<Solver*>(s)->solver.grid_report();

@@ -111,8 +111,10 @@ struct KrylovSolver::Impl {
   DeviceArray<kh_tail_level> tail_table;
   // The multi-workgroup V-cycle: levels [grid_first, end) run as one
   // KH_GRID_CYCLE launch (0: off), in place of the tail, when the tail is
-  // automatic. grid_request < 0 picks the level by the rule in pick_grid.
+  // automatic. grid_request < 0 picks the level by the rule in pick_grid;
+  // grid_off: the caller wants none, whatever is picked or timed.
   int grid_request = -1;
+  bool grid_off = false;
   int grid_first = 0;
   int grid_limit_us = 2000;  // how long its workgroups wait for each other
   GridPlan grid_plan;
@@ -628,7 +630,7 @@ struct KrylovSolver::Impl {
     grid_spread = grid_ctl.download()[KH_GRID_CTL_SPREAD] == KH_GRID_MAX_PARTS;
   }
   void pick_grid() {
-    if (grid_request == 0) return;
+    if (grid_request == 0 || grid_off) return;
     if (grid_request > 0) {
       if (plan_grid_at(std::size_t(grid_request), grid_plan)) use_grid(grid_request);
       return;
@@ -1526,6 +1528,7 @@ int KrylovSolver::set_tail(int first) {
   return impl_->tail_first;
 }
 int KrylovSolver::tail_level() const { return impl_->tail_first; }
+int KrylovSolver::grid_level() const { return impl_->grid_first; }
 int KrylovSolver::set_grid(int first, int limit_us) {
   Impl& I = *impl_;
   KA_REQUIRE(limit_us >= 0, "AMG: the multi-workgroup cycle's wait must not be negative");
@@ -1536,6 +1539,7 @@ int KrylovSolver::set_grid(int first, int limit_us) {
   }
   I.grid_request = first;
   I.grid_asked = first > 0;
+  I.grid_off = first == 0;
   I.grid_limit_us = limit_us;
   if (first != 0) I.tail_request = -1;
   I.plan_tail();
@@ -1553,7 +1557,8 @@ void KrylovSolver::set_grid_polls(int polls) {
 
 // The coarse-tail autotuner (no reference counterpart): times `repeats`
 // V-cycles for each admissible first level of the tail, and for none, keeps
-// the fastest and returns it. Every choice gives bitwise the same iterates
+// the fastest and returns it (-1: the multi-workgroup cycle, timed beside it
+// unless the caller turned it off). Every choice gives bitwise the same iterates
 // (the tail computes each row as the per-level launches do), so it picks
 // only the launch structure: per-level launches are latency-bound below a
 // few thousand rows, the one-workgroup tail is compute-bound on one CU, and
@@ -1709,7 +1714,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
   // The multi-workgroup cycle from each level whose plan fits, in the tail's place.
   int best_grid = 0;
   for (std::size_t i = 1; i < I.levels.size(); ++i) {
-    if (!I.grid_allowed(i)) continue;
+    if (I.grid_off || !I.grid_allowed(i)) continue;
     I.tail_request = -1;
     I.grid_request = int(i);
     I.plan_tail();
@@ -1727,7 +1732,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
   I.grid_request = best_grid;
   I.tail_request = best;
   I.plan_tail();
-  return I.tail_first;
+  return I.grid_first > 0 ? -1 : I.tail_first;
 }
 int KrylovSolver::host_waits() const { return impl_->waits; }
 int KrylovSolver::set_direct(Index rows) { return impl_->set_direct(rows); }
@@ -1849,10 +1854,10 @@ std::string KrylovSolver::plan() const {
         << (impl_->coarse_sweeps_mode == 0                                      ? "sweep launches"
             : impl_->coarse_sweeps_mode == 2 && L.back().resident_cap > 0 ? "register-resident sweeps"
                                                                             : "one-workgroup sweeps");
-  out << "; tail from level " << impl_->tail_first;
+  if (!impl_->grid_on()) out << "; tail from level " << impl_->tail_first;
   if (impl_->grid_first > 0) {
     const GridPlan& g = impl_->grid_plan;
-    out << ", multi-workgroup cycle from level " << impl_->grid_first << " (" << g.parts << " workgroups, " << g.grid
+    out << (impl_->grid_on() ? "; " : ", ") << "multi-workgroup cycle from level " << impl_->grid_first << " (" << g.parts << " workgroups, " << g.grid
         << " of " << g.count << " levels shared, row sums";
     for (int k = 0; k < g.count; ++k) out << (k ? "," : " ") << (g.table[std::size_t(k)].mode ? "split" : "whole");
     out << ")";

@@ -107,6 +107,7 @@ class KrylovSolver {
   // times it rests for 256 solves. Returns the level in use, 0 for none
   // (iterates are the same).
   int set_grid(int first, int limit_us);
+  int grid_level() const;
   // How often a barrier between those workgroups polls before it gives up
   // (default 2^21): the solve that finds one given up throws, and the cycle is
   // off until set_grid or set_tail(-1) asks for it again.
@@ -114,9 +115,11 @@ class KrylovSolver {
   // Launches of that cycle so far: by its workgroups together, by one alone,
   // and with a barrier given up.
   std::array<Index, 3> grid_report() const;
-  // Times `repeats` V-cycles per admissible tail level (and none) on the
-  // refreshed operator and keeps the fastest; returns it. Identical iterates
-  // either way. No reference counterpart.
+  // Times `repeats` V-cycles per admissible tail level (and none), and the
+  // multi-workgroup cycle unless set_grid(0) turned it off, on the refreshed
+  // operator and keeps the fastest. Returns the tail's level, 0 for none, or -1
+  // for that cycle (its level: grid_level). Identical iterates either way. No
+  // reference counterpart.
   int autotune_tail(const DeviceCsr& a, int repeats);
   // Restart length of the FGMRES kinds (default 30, at most 63).
   void set_restart(int m);

@@ -191,6 +191,34 @@ def test_a_cycle_that_does_not_meet_rests(device):
     assert "resting" not in solver.plan()
 
 
+def test_the_tuner_says_what_it_chose(device):
+    """autotune_tail returns -1 exactly where it chose the cycle, and that given
+    to set_tail chooses it again; a cycle turned off by the caller is neither
+    tuned in nor brought back by the automatic tail."""
+    a = oracle.poisson(30, 28, 26)
+    host = kutta_amd.CsrMatrixHost(a.row_ptr, a.col, a.diag, a.val)
+    matrix = kutta_amd.upload(device, host)
+    solver = kutta_amd.make_amg_solver(SolverKind.AmgPcg, device, host, AmgOptions())
+    solver.refresh(matrix)
+    tail = solver.set_tail(-1)
+    assert tail >= 1 and solver.grid_level >= 1 and f"tail from level {tail}" not in solver.plan()
+    for _ in range(2):
+        chosen = solver.autotune_tail(matrix, 2)
+        assert (chosen == -1) == (solver.grid_level > 0) == ("multi-workgroup" in solver.plan())
+        kept = solver.grid_level
+        if kept:
+            assert solver.set_grid(kept) == kept
+        assert solver.set_tail(chosen) == (tail if chosen < 0 else chosen)
+        assert (solver.grid_level > 0) == (kept > 0)
+        solver.set_tail(0)  # the tuner times the cycle again after a tail was set
+    assert solver.set_grid(0) == 0
+    assert solver.autotune_tail(matrix, 2) >= 0
+    assert solver.grid_level == 0 and "multi-workgroup" not in solver.plan()
+    assert solver.set_tail(-1) == tail and solver.grid_level == 0
+    assert f"tail from level {tail}" in solver.plan()
+    assert solver.set_grid(-1) >= 1
+
+
 class Level(C.Structure):
     _fields_ = [(k, C.c_void_p) for k in ("row_ptr", "col", "val", "inverse", "member_offsets", "members", "aggregate",
                                           "place", "slot", "local_col", "x", "w", "b")] + [
