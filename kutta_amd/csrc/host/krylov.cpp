@@ -212,7 +212,7 @@ struct KrylovSolver::Impl {
     if (!on)
       for (auto& l : levels) l.val16 = DeviceArray<std::uint16_t>();
   }
-  DeviceArray<double> dense_inverse, dense_scratch;
+  DeviceArray<double> dense_inverse;
   // Lazy dense refresh (no reference counterpart): with a tolerance > 0 a
   // refresh keeps the inverse while the level's values stay within that
   // relative l2 distance of the values it was computed from (`dense_basis`);
@@ -226,7 +226,6 @@ struct KrylovSolver::Impl {
     direct_ready = false;
     dense_basis = DeviceArray<float>();
     dense_inverse = DeviceArray<double>();
-    dense_scratch = DeviceArray<double>();
     if (rows <= 0) {
       plan_tail();
       return 0;
@@ -242,7 +241,6 @@ struct KrylovSolver::Impl {
     KA_REQUIRE(direct_level > 0, "AMG: no coarse level has at most " + std::to_string(rows) + " rows");
     const std::size_t nc = std::size_t(levels[direct_level].rows);
     dense_inverse = DeviceArray<double>(dev, nc * nc);
-    dense_scratch = DeviceArray<double>(dev, 64 * 64);  // the pivot block's inverse
     plan_tail();
     return direct_level;
   }
@@ -750,7 +748,7 @@ struct KrylovSolver::Impl {
         invert = !(dense_staleness <= dense_tolerance);
       }
       if (invert) {
-        dev.launch(KH_DENSE_INVERT, c.n_rows, {c.row_ptr, c.col, c.val, dense_inverse, dense_scratch});
+        dev.launch(KH_DENSE_INVERT, c.n_rows, {c.row_ptr, c.col, c.val, dense_inverse, status});  // no scratch used
         if (dense_tolerance > 0) {
           if (dense_basis.size() != std::size_t(c.nnz)) dense_basis = DeviceArray<float>(dev, c.nnz);
           dev.copy(dense_basis.data(), c.val, sizeof(float) * std::size_t(c.nnz));
