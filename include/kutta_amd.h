@@ -373,7 +373,8 @@ int64_t ka_learned_parameter_count(int layers); /* -1 outside 1..4 */
 int ka_learned_create(void* dev, int layers, uint64_t seed, void** out);
 void ka_learned_destroy(void* net);
 /* Node features and neighbour weights of a symmetric operator with positive
- * diagonal (a ka_matrix handle); again after its values change. */
+ * diagonal (a ka_matrix handle); again after its values change. The network
+ * reads the matrix's pattern until it has another graph: free it after that. */
 int ka_learned_set_graph(void* net, void* matrix);
 int ka_learned_set_parameters(void* net, const float* theta, int64_t count);
 int ka_learned_parameters(void* net, float* theta, int64_t count);

@@ -1686,6 +1686,7 @@ class LearnedNetwork:
 
     def set_graph(self, a: CsrMatrix) -> None:
         _check_host(host_lib().ka_learned_set_graph(self.handle, a.handle))
+        self._graph = a  # the network reads its pattern from now on
 
     def set_parameters(self, theta) -> None:
         t = np.ascontiguousarray(theta, dtype=np.float32)
