@@ -514,8 +514,8 @@ typedef struct kh_grid_part {
 /* Words of a control block that INIT sets and its owner may change between
  * launches: the polls a barrier makes before it gives up (2^21), and the device
  * address (64 bits) of KH_GRID_REPORT_WORDS counters that CYCLE adds to (0: none):
- * launches in which a barrier gave up, that ran together, and in which one
- * workgroup worked alone. HOME is the XCD whose workgroups work, at first the
+ * barriers given up by a workgroup, launches that ran together, and launches in
+ * which one workgroup worked alone. HOME is the XCD whose workgroups work, at first the
  * one that INIT ran on, and SPREAD how many workgroups of a launch of
  * 8 KH_GRID_MAX_PARTS found themselves there: where it is KH_GRID_MAX_PARTS,
  * launches go round-robin over 8 XCDs, as CYCLE's workgroups need to meet. */

@@ -64,13 +64,10 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // kh_grid_gather.hpp uses it; the limit is in ticks of the 100 MHz clock.
 struct GridCtl {
   unsigned *arrived, *settled, *bar, *home, *left;
-  unsigned polls;
-  int* report;
   long limit;
   long long start = 0;
   __device__ GridCtl(unsigned* w, long limit_ticks)
-      : arrived(w), settled(w + 32), bar(w + 64), home(w + KH_GRID_CTL_HOME), left(w + 128),
-        polls(w[KH_GRID_CTL_POLLS]), report(*reinterpret_cast<int**>(w + KH_GRID_CTL_REPORT)), limit(limit_ticks) {}
+      : arrived(w), settled(w + 32), bar(w + 64), home(w + KH_GRID_CTL_HOME), left(w + 128), limit(limit_ticks) {}
   __device__ static unsigned add(unsigned* p, unsigned v) {
     return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -91,7 +88,10 @@ struct GridCtl {
     for (unsigned* p : {bar, left, settled, arrived})
       __hip_atomic_store(p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  // Through a global pointer: behind a flat atomic the cycle's loops wait for
+  // more than they need, 0.1 us a sweep.
   __device__ void count(int what) const {
+    GLOBAL int* report = (GLOBAL int*)*reinterpret_cast<int**>(arrived + KH_GRID_CTL_REPORT);
     if (report != nullptr) __hip_atomic_fetch_add(report + what, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 };
@@ -100,7 +100,16 @@ struct GridCtl {
 // passes the same barriers, so the wait ends. It is bounded all the same: after
 // `polls` polls of some 0.3 us each a member gives up, which opens this and the
 // launch's later barriers to all and is reported, since the iterate is wrong.
+// What this needs is kept in LDS: the cycle is short of scalar registers.
 constexpr unsigned kGivenUp = 1u << 31, kBarrierPolls = 1u << 21;
+struct GridWait {
+  GridPlace place;
+  unsigned polls, given_up;
+};
+__device__ __forceinline__ GridWait& grid_wait() {
+  __shared__ GridWait w;
+  return w;
+}
 __device__ __forceinline__ void grid_sync(const GridCtl& c, int parts, unsigned& passed) {
   stores_done();
   __syncthreads();
@@ -109,10 +118,11 @@ __device__ __forceinline__ void grid_sync(const GridCtl& c, int parts, unsigned&
     GLOBAL unsigned* bar = (GLOBAL unsigned*)c.bar;
     __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned polls = 0, seen;
-    while ((seen = ctl_load(c.bar)) < passed && polls < c.polls) ++polls;
-    if (seen < passed &&
-        (__hip_atomic_fetch_or(bar, kGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kGivenUp) == 0)
-      c.count(KH_GRID_REPORT_GIVEN_UP);
+    while ((seen = ctl_load(c.bar)) < passed && polls < grid_wait().polls) ++polls;
+    if (seen < passed) {
+      __hip_atomic_fetch_or(bar, kGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      grid_wait().given_up = 1;
+    }
   }
   __syncthreads();
 }
@@ -507,18 +517,23 @@ __device__ __forceinline__ void member_cycle(const CycleArgs& A, const GridCtl& 
 
 __global__ void __launch_bounds__(kGridThreads) k_grid_cycle(const CycleArgs A) {
   if (A.status[0] != 0) return;
-  __shared__ GridPlace place;
   GridCtl ctl(A.ctl, long(A.limit_us) * 100);
-  if (threadIdx.x == 0) place = grid_enter(ctl, gridDim.x, A.parts, xcc_id() == ctl_load(ctl.home));
+  if (threadIdx.x == 0) {
+    const unsigned polls = ctl_load(A.ctl + KH_GRID_CTL_POLLS);
+    grid_wait() = {grid_enter(ctl, gridDim.x, A.parts, xcc_id() == ctl_load(ctl.home)), polls, 0};
+  }
   __syncthreads();
+  const GridPlace place = grid_wait().place;
   const GridRole role = GridRole(__builtin_amdgcn_readfirstlane(int(place.role)));
-  // Counted at once, so that the cycle hides it.
-  if (threadIdx.x == 0 && role == GridRole::Solo) ctl.count(KH_GRID_REPORT_ALONE);
-  if (threadIdx.x == 0 && role == GridRole::Member && place.rank == 0) ctl.count(KH_GRID_REPORT_TOGETHER);
   if (role == GridRole::Member) member_cycle(A, ctl, __builtin_amdgcn_readfirstlane(place.rank));
   else if (role == GridRole::Solo) solo_cycle(A);
   __syncthreads();
-  if (threadIdx.x == 0) grid_leave(ctl, gridDim.x);
+  if (threadIdx.x == 0) {
+    if (role == GridRole::Solo) ctl.count(KH_GRID_REPORT_ALONE);
+    if (role == GridRole::Member && place.rank == 0) ctl.count(KH_GRID_REPORT_TOGETHER);
+    if (grid_wait().given_up) ctl.count(KH_GRID_REPORT_GIVEN_UP);
+    grid_leave(ctl, gridDim.x);
+  }
 }
 
 // Clears a control block and records the XCD of this workgroup as its home.
