@@ -27,9 +27,9 @@ struct GridPlan {
 // Plans levels patterns[0..] (the first is where the launch starts) over
 // `parts` workgroups. The levels of at most KH_GRID_BOTTOM_ROWS rows at the
 // end belong to the first workgroup. Returns false where the plan does not
-// fit: a member's share of all its levels, its two widest windows and the
-// terms of the levels that form them must lie in KH_GRID_POOL_WORDS words of
-// LDS.
+// fit: a member's share of all its levels, the launch's widest window and the
+// terms of its largest level that forms them must lie in KH_GRID_POOL_WORDS
+// words of LDS, with the first member's bottom levels and their iterates.
 bool plan_grid(const std::vector<const CsrHost*>& patterns, int parts, GridPlan& plan);
 
 }  // namespace kutta_amd

@@ -585,19 +585,24 @@ struct KrylovSolver::Impl {
 
   // ---- the multi-workgroup V-cycle (KH_GRID_CYCLE)
   // By itself it takes over from the first level, at least two before the end,
-  // whose plan fits the LDS of 16 workgroups. Whole solves of tetrahedral
-  // pressure problems, V(5,5), ms:
-  //     first level's rows           none  tail only   8      16      32
-  //     1.0M cells, 17,004          18.34    18.34     -       -    16.86
-  //                  5,023                             -    17.03   17.35
-  //                  2,017                           17.19  17.24   17.54
-  //     78k cells,  19,808           5.75     5.81     -       -     5.15
-  //                  5,138                            5.03   5.01    5.21
-  //     10k cells,   2,611           4.59     3.97    2.63   2.64    2.69
-  //                    681                            2.94   2.92    2.96
-  // so 8 or 16 workgroups do alike, and 32, which hold more, pay only where the
-  // autotuner finds so or a caller asks. A last level by itself (15,292 rows, 4
-  // sweeps a visit under a K-cycle) took 19.25 against 18.81.
+  // whose plan fits the LDS of 16 workgroups. Solves of tetrahedral pressure
+  // problems, V(5,5), ms (repeats differ by up to 2% at 10k and 78k cells, by 4%
+  // at 1.0M; "tail": the best the automatic tail's rule allows):
+  //     first level's rows           none   tail     8      16      32
+  //     10k cells,   2,611           4.57   3.98   2.60    2.60    2.65
+  //                    681                         2.87    2.92    2.94
+  //     78k cells,  19,808           5.81   7.18     -       -     5.10
+  //                  5,138                         5.00    4.94    5.26
+  //                  1,397                         4.97    5.02    5.31
+  //     1.0M cells, 17,004          18.29  23.70     -       -    17.06
+  //                  5,023                           -    17.15   17.21
+  //                  2,017                        17.40   17.40   17.45
+  //                  1,067                        17.77   17.78   17.75
+  // so 8 or 16 workgroups do alike, and 32, which hold more, within the noise of
+  // the next level on 16 at 1.0M cells and worse at 78k: they are for the
+  // autotuner and for callers that ask. A last level by itself (15,292 rows, 4
+  // sweeps a visit under a K-cycle) took 19.25 against 18.81: only the autotuner
+  // tries it.
   static constexpr Index kGridAutoRows = 24576;
   static constexpr int kGridParts = 16;
   bool grid_allowed(std::size_t first) const {
@@ -1677,10 +1682,8 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
     }
     l.prolong_mode = pick;
   }
-  // The coarsest level's sweeps: launch by launch or in one workgroup. The
-  // one-workgroup form that reads the operator once (set_plan form 2) is not
-  // a candidate: measured, it never beat the launches by more than noise on
-  // the benchmark hierarchies, and as a candidate it was picked by noise.
+  // The coarsest level's sweeps: launch by launch, in one workgroup or, where
+  // the level has a resident partition, in one that reads the operator once.
   if (I.coarse_sweeps_fit(I.levels.size() - 1)) {
     double fastest = 0;
     int pick = 0;

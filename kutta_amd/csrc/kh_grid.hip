@@ -7,11 +7,11 @@
 // coarsest. One workgroup (the coarse tail) pays no launches but computes on
 // one CU. Here the rows of every level are split over `parts` workgroups that
 // stay on one XCD and keep their operators in LDS for the whole cycle. A sweep
-// then takes 2.5 us (1.3 the rows' serial sums, 0.6 the barrier, 0.4 the
-// window); a pressure solve (AMG-PCG, V(5,5)) of 10,368 cells went from 4.20 to
-// 2.86 ms, of 78,246 from 6.24 to 5.42, of 998,250 from 20.28 to 17.87. 512 or
-// 256 threads instead of 1024 measured the same on small levels, slower on
-// large.
+// then takes 2.3 to 2.5 us (1.3 the rows' serial sums, 0.6 the barrier, 0.4 the
+// window); a pressure solve (AMG-PCG, V(5,5)) of 10,368 cells takes 2.6 ms and
+// without it 4.6, of 78,246 4.9 and 5.8, of 998,250 17.3 and 18.3 (the rule
+// that picks the first level has the whole table). 512 or 256 threads instead
+// of 1024 measured the same on small levels, slower on large.
 //
 // Exchange: a sweep's new values go out as write-through stores and come in,
 // after a barrier over the workgroups, as one coalesced window of the iterate

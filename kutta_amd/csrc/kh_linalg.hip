@@ -1633,13 +1633,19 @@ unsigned reduce_grid(int n) {
   return blocks;
 }
 // The tickets of a reduction over g workgroups, or null where a launch of its
-// own finishes it. The last workgroup saves a launch of some 3.5 us (and the
-// gap before it) but the ticket counters take a time of their own: with all
-// reductions finished that way against none, batched BiCGStab iterations of
-// 594 workgroups a lane went from 51.8 to 47.3 us, SIMPLEC iterations of 4
-// workgroups from 3.14 to 2.90 ms; of 2000 workgroups they took 4.5 ms
-// against 4.3 with launches above this line, and a solve of 3900 workgroups
-// 17.8 ms against 17.5.
+// own finishes it. In kernel time tickets cost more than that launch at every
+// size; row kernel and ending, replayed from a graph, us, launch / tickets:
+//     workgroups            60           1,000         4,000
+//     p.q, alpha        5.7 /  6.7     8.5 /  9.8    19.6 / 20.8
+//     r.r, check        4.5 /  5.4     5.8 /  7.2    10.0 / 13.1
+//     t.t, t.s, 3 lanes 7.5 /  7.7    18.3 / 19.2    48.7 / 53.2
+// What they save is the host's launch, which loops launched kernel by kernel
+// wait for while kernels are short. Three systems by batched BiCGStab, ms:
+//     workgroups    256   512   768  1,024  1,536  2,048  3,072
+//     launch       4.49  5.28  5.74   6.17   7.67   8.60  10.28
+//     tickets      4.00  4.77  5.44   6.00   7.52   8.75  10.69
+// Whole PCG solves replayed from a graph (41 and 306 workgroups) are within 1%
+// either way, so the line is the same there.
 constexpr unsigned kTicketBlocks = 1024;
 unsigned* tickets(kh_device* d, unsigned g) { return g <= kTicketBlocks ? d->tickets : nullptr; }
 #define FINISH dim3(1), dim3(kBlock), 0, d->stream
