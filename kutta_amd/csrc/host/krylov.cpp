@@ -138,7 +138,10 @@ struct KrylovSolver::Impl {
   int grid_missed = 0;   // of this solve
   int grid_rest = 0;     // solves left without the cycle, this one among them
   bool grid_spread = false;  // launches go over the XCDs as the cycle needs
-  bool grid_on() const { return grid_first > 0 && !coarse_bf16 && grid_rest == 0; }
+  // The level it is planned from (0: none; it has no bfloat16 form), and
+  // whether cycles run it now.
+  int grid_level() const { return coarse_bf16 ? 0 : grid_first; }
+  bool grid_on() const { return grid_level() > 0 && grid_rest == 0; }
 
   Impl(HipDevice& d, SolverKind k, const CsrHost& a, const AmgOptions& o)
       : dev(d), kind(k), options(o),
@@ -1531,7 +1534,7 @@ int KrylovSolver::set_tail(int first) {
   return impl_->tail_first;
 }
 int KrylovSolver::tail_level() const { return impl_->tail_first; }
-int KrylovSolver::grid_level() const { return impl_->grid_first; }
+int KrylovSolver::grid_level() const { return impl_->grid_level(); }
 int KrylovSolver::set_grid(int first, int limit_us) {
   Impl& I = *impl_;
   KA_REQUIRE(limit_us >= 0, "AMG: the multi-workgroup cycle's wait must not be negative");
@@ -1546,7 +1549,7 @@ int KrylovSolver::set_grid(int first, int limit_us) {
   I.grid_limit_us = limit_us;
   if (first != 0) I.tail_request = -1;
   I.plan_tail();
-  return I.grid_first;
+  return I.grid_level();
 }
 std::array<Index, 3> KrylovSolver::grid_report() const {
   const auto host = impl_->status.download();
@@ -1733,7 +1736,7 @@ int KrylovSolver::autotune_tail(const DeviceCsr& a, int repeats) {
   I.grid_request = best_grid;
   I.tail_request = best;
   I.plan_tail();
-  return I.grid_first > 0 ? -1 : I.tail_first;
+  return I.grid_level() > 0 ? -1 : I.tail_first;
 }
 int KrylovSolver::host_waits() const { return impl_->waits; }
 int KrylovSolver::set_direct(Index rows) { return impl_->set_direct(rows); }
@@ -1856,7 +1859,7 @@ std::string KrylovSolver::plan() const {
             : impl_->coarse_sweeps_mode == 2 && L.back().resident_cap > 0 ? "register-resident sweeps"
                                                                             : "one-workgroup sweeps");
   if (!impl_->grid_on()) out << "; tail from level " << impl_->tail_first;
-  if (impl_->grid_first > 0) {
+  if (impl_->grid_level() > 0) {
     const GridPlan& g = impl_->grid_plan;
     out << (impl_->grid_on() ? "; " : ", ") << "multi-workgroup cycle from level " << impl_->grid_first << " (" << g.parts << " workgroups, " << g.grid
         << " of " << g.count << " levels shared, row sums";

@@ -216,7 +216,13 @@ def test_the_tuner_says_what_it_chose(device):
     assert solver.grid_level == 0 and "multi-workgroup" not in solver.plan()
     assert solver.set_tail(-1) == tail and solver.grid_level == 0
     assert f"tail from level {tail}" in solver.plan()
-    assert solver.set_grid(-1) >= 1
+    first = solver.set_grid(-1)
+    assert first >= 1
+    solver.set_coarse_bf16(True)  # the cycle has no such form: the tail runs
+    assert solver.grid_level == 0 and "multi-workgroup" not in solver.plan()
+    assert f"tail from level {tail}" in solver.plan()
+    solver.set_coarse_bf16(False)
+    assert solver.grid_level == first
 
 
 class Level(C.Structure):
